@@ -10,6 +10,10 @@
 // The value of x (in an SGPR: "s", a VGPR: "v") passed through an empty asm: expressions
 // formed from it afterwards are new to the compiler and are not merged with earlier ones.
 #define LQMC_OPAQUE(x, reg) asm volatile("" : "+" reg(x))
+// Issue priority of the calling wavefront on its SIMD (0..3).
+#define LQMC_WAVE_PRIO(p) __builtin_amdgcn_s_setprio(p)
+#else
+#define LQMC_WAVE_PRIO(p) ((void)0)
 #endif
 #include <stdint.h>
 

@@ -685,13 +685,18 @@ __global__ __launch_bounds__(QF_THREADS) void k_trsm_perm(const TrsmTask* __rest
 //   1. applies Q_P^T = I - V T^T V^T of every panel P left of its strip, from LDS, on the
 //      matrix cores: W = V^T X, W' = T^T W, X -= V W' (the accumulator layout of X is the
 //      operand layout of these products, so nothing is transposed);
-//   2. factors its own panel: the strip goes through LDS into a row-per-lane layout (rows
-//      j0 + lane + 64i), one wavefront reduction per column (Householder, no pivoting beyond
-//      the pre-pivot: the columns of the UDV chain are graded, and sorting them by norm once
-//      is what keeps the factorisation accurate), then V and T go to LDS for the others,
-//      the reflectors to A, T to Tt, |diag R| to D, and the strip's columns of D^-1 R (final:
+//   2. factors its own panel in that layout (Householder, no pivoting beyond the pre-pivot: the
+//      columns of the UDV chain are graded, and sorting them by norm once is what keeps the
+//      factorisation accurate): V goes to LDS for the others, and while they form V^T X the
+//      wavefront forms T from the V in its registers; then, off the panel chain, the
+//      reflectors go to A, T to Tt, |diag R| to D, and the strip's columns of D^-1 R (final:
 //      later panels touch only columns right of it) to W;
 //   3. only meets the workgroup barriers of the remaining panels (its registers are free).
+// Bound by the latency of the panel chain, 16 dependent column steps per panel (about 1400 cycles
+// each up to 128 rows).  Factoring in the accumulator layout, with T off the chain, instead of
+// through a row-per-lane copy of the strip: 139 -> 59 us at N = 64 (k_qr_small), 272 -> 154 us at
+// N = 117 (32 chains), 635 -> 589 us at N = 256 (64 chains; two passes over the pivot column in
+// LDS, as the strip leaves no registers for it), all with the same results bit for bit.
 // The right half receives the left half's panels (reflectors in A, T in Tt, D) through global
 // memory behind a per-matrix release counter, hand[2 task] = panels published; the left half
 // writes W (which both halves read at the start) only after the right half has released
@@ -731,12 +736,14 @@ __device__ inline void qo_wait(unsigned* c, unsigned after, ChainState* st, int 
 }
 
 // Q_P^T applied to one strip held in registers (rows j0 = 16 P .. 16 NS - 1; the panel's V,
-// explicit with unit diagonal and zeros above it, in vbuf; T in tbuf).
-__device__ inline void qo_apply(qo_acc_t (&acc)[16], const double* vbuf, const double* tbuf, int NS, int P) {
+// explicit with unit diagonal and zeros above it, in vbuf; T in tbuf), NT >= NS row tiles held:
+// V^T X, which needs V alone, then X -= V (T^T (V^T X)).
+template <int NT>
+__device__ inline qr_v4d qo_apply_vt(const qo_acc_t (&acc)[NT], const double* vbuf, int NS, int P) {
   const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
   qr_v4d wt = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-  for (int t = 0; t < 16; ++t) {
+  for (int t = 0; t < NT; ++t) {
     if (t < P || t >= NS) continue;
     double a[4];
 #pragma unroll
@@ -744,11 +751,17 @@ __device__ inline void qo_apply(qo_acc_t (&acc)[16], const double* vbuf, const d
 #pragma unroll
     for (int v = 0; v < 4; ++v) wt = qr_mma(a[v], acc[t][v], wt);
   }
+  return wt;
+}
+template <int NT>
+__device__ inline void qo_apply_v(qo_acc_t (&acc)[NT], const double* vbuf, const double* tbuf, qr_v4d wt, int NS,
+                                  int P) {
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
   qr_v4d w2 = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
   for (int s = 0; s < 4; ++s) w2 = qr_mma(tbuf[(4 * s + lk) * 16 + li], wt[s], w2);
 #pragma unroll
-  for (int t = 0; t < 16; ++t) {
+  for (int t = 0; t < NT; ++t) {
     if (t < P || t >= NS) continue;
     double a[4];
 #pragma unroll
@@ -756,6 +769,10 @@ __device__ inline void qo_apply(qo_acc_t (&acc)[16], const double* vbuf, const d
 #pragma unroll
     for (int s = 0; s < 4; ++s) acc[t] = qr_mma(a[s], w2[s], acc[t]);
   }
+}
+template <int NT>
+__device__ inline void qo_apply(qo_acc_t (&acc)[NT], const double* vbuf, const double* tbuf, int NS, int P) {
+  qo_apply_v<NT>(acc, vbuf, tbuf, qo_apply_vt<NT>(acc, vbuf, NS, P), NS, P);
 }
 
 // Q formation for N <= 256 with the column block held in registers: one 256-thread workgroup
@@ -800,7 +817,7 @@ __global__ __launch_bounds__(QF_THREADS, 2) void k_qr_formq_onchip(const QrTask*
       tbuf[e] = (i < w && j < w) ? tk.Tt[(size_t)P * 256 + j * 16 + i] : 0.0;
     }
     __syncthreads();
-    if (cs >= P && cs < NS) qo_apply(acc, vbuf, tbuf, NS, P);
+    if (cs >= P && cs < NS) qo_apply<16>(acc, vbuf, tbuf, NS, P);
   }
   if (c < c1)
 #pragma unroll
@@ -902,112 +919,352 @@ __global__ __launch_bounds__(QF_THREADS, 2) void k_trsm_onchip(const TrsmTask* _
 
 size_t trsm_onchip_shmem() { return sizeof(double) * (16 * (size_t)TO_LD + 16 * QF_COLS); }
 
+// LDS of k_qr_onchip and k_qr_small.
 struct QoShared {
-  double *sbuf, *vbuf, *tbuf, *ssc, *red, *dbuf, *taus;
-  const int* perm;
+  double *vbuf, *tbuf;  // [2][rows][17] V and [2][16][16] T of panels of either parity
+  double *xbuf, *rbuf;  // [rows + 16] pivot column by tile (last: unread), [16][16] the panel's rows of R
+  double *ssc, *taus;   // [16][16] S = V^T V, [16] reflector coefficients
+  double* dbuf;         // [rows] |diag R|
+  int vs;               // doubles of one V
 };
 
-// Step 2 for panel P (rows j0..N-1, w columns) of the calling wavefront's strip.  hand: the
-// matrix's two hand-over counters, or null when one workgroup holds the whole matrix;
-// left: the calling workgroup is the left half of a split matrix.
-__device__ void qo_factor(qo_acc_t (&acc)[16], const QrTask& tk, const QoShared& sh, int N, int P, int w,
-                          unsigned* hand, bool left, ChainState* st, bool& broken, bool& zero_pivot) {
-  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
-  const int j0 = P << 4;
-  double* sbuf = sh.sbuf;
-  // the whole strip to LDS; the registers are not used again
+// a / b as the compiler's FP64 division forms it, without its scaling of operands and result: the
+// same quotient for operands and quotients well inside the exponent range.
+__device__ inline double qo_div(double a, double b) {
+#ifdef LQMC_CPU_EMU
+  return a / b;
+#else
+  double r = __builtin_amdgcn_rcp(b);
+  r = fma(fma(-b, r, 1.0), r, r);
+  r = fma(fma(-b, r, 1.0), r, r);
+  const double q = a * r;
+  return fma(fma(-b, q, a), r, q);
+#endif
+}
+// sqrt(x) likewise, x well inside the exponent range.
+__device__ inline double qo_sqrt(double x) {
+#ifdef LQMC_CPU_EMU
+  return sqrt(x);
+#else
+  const double r = __builtin_amdgcn_rsq(x);
+  double s = x * r, h = r * 0.5;
+  const double e = fma(-h, s, 0.5);
+  s = fma(s, e, s);
+  h = fma(h, e, h);
+  s = fma(fma(-s, s, x), h, s);
+  return fma(fma(-s, s, x), h, s);
+#endif
+}
+
+// One panel's factorisation state of a lane (its column c = l % 16 of the panel).
+struct QoPanel {
+  qo_acc_t pt;   // copy of the panel's diagonal tile (tile P of the strip)
+  double scal;   // 1 / (alpha - beta): V = u scal below the diagonal
+  double beta;   // R[c][c]
+  bool zero;     // a pivot column was zero
+};
+
+// f(t, x of tile t) over the strip's tiles, x the pivot column's entries from LDS.  Up to 8 tiles:
+// all of them, x held in registers by the caller.  16 tiles: the tile pairs from that of tile P on,
+// x read one pair ahead of its use; the scheduling fences keep the compiler from reading all of it
+// first (its registers would displace the strip's).
+template <int NT, typename F>
+__device__ __attribute__((always_inline)) inline void qo_tiles(const qo_acc_t* xl, const qo_acc_t (&xr)[NT], int P,
+                                                               F f) {
+  if constexpr (NT <= 8) {
 #pragma unroll
-  for (int t = 0; t < 16; ++t)
+    for (int t = 0; t < NT; ++t) f(t, xr[t]);
+  } else {
+    qo_acc_t x[NT];
+    x[0] = xl[0];
+    x[1] = xl[4];
 #pragma unroll
-    for (int v = 0; v < 4; ++v) sbuf[(16 * t + lk + 4 * v) * QO_PS + li] = acc[t][v];
-  qr_wave_sync();
-  double x[4][16];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = j0 + lane + 64 * i;
-    const bool ok = r < N;
-#pragma unroll
-    for (int c = 0; c < 16; ++c) x[i][c] = ld0(sbuf, (size_t)r * QO_PS + c, ok);
-  }
-#pragma unroll
-  for (int q = 0; q < 16; ++q) {
-    if (q < w) {
-      const int j = j0 + q;
-      // s_c = x^T col_c over rows >= j for the column x = col_q (s_q = |x|^2), into red
-      {
-        double part[16];
-#pragma unroll
-        for (int c = 0; c < 16; ++c) part[c] = 0.0;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int r = j0 + lane + 64 * i;
-          const double xv = r >= j ? x[i][q] : 0.0;  // rows >= N hold zeros
-#pragma unroll
-          for (int c = q; c < 16; ++c) part[c] += xv * x[i][c];
-        }
-        qr_wave_colsum<16>(part, sh.red, lane);
+    for (int g = 0; g < NT / 2; ++g) {
+      if (2 * g + 2 < NT) {
+        x[2 * g + 2] = xl[8 * g + 8];
+        x[2 * g + 3] = xl[8 * g + 12];
       }
-      const double alpha = qo_readlane(x[0][q], q);  // row j is lane q's first row
-      const double xx = sh.red[q];
-      const double nrmv = sqrt(xx > 0.0 ? xx : 0.0);
-      double beta, tau, scal;
-      if (nrmv == 0.0) {
-        beta = 0.0; tau = 0.0; scal = 0.0;
-        zero_pivot = true;
+      if (2 * g + 1 >= P) {
+        f(2 * g, x[2 * g]);
+        f(2 * g + 1, x[2 * g + 1]);
+      }
+      qr_sched_fence();
+    }
+  }
+}
+
+// The 64 row sequences of a panel column (s[t % 4][v] of lanes l, l ^ 16, l ^ 32, l ^ 48) combined, in
+// every lane.  The order is fixed: sequences p, p + 32; then + 16; then within neighbours, quads, and
+// the four quads as (0 + 3) + (2 + 1).
+template <int NT>
+__device__ __attribute__((always_inline)) inline double qo_combine(const qo_acc_t (&s)[4]) {
+  qo_acc_t u;
+  if constexpr (NT == 2) u = s[0] + s[1];
+  else u = (s[0] + s[2]) + (s[1] + s[3]);
+  double u0 = u[0], u1 = u[1], u2 = u[2], u3 = u[3];
+  qr_swap<16>(u0, u3);
+  qr_swap<16>(u2, u1);
+  double a = u0 + u3, b = u2 + u1;
+  qr_swap<32>(a, b);
+  double y = a + b;
+  b = y;
+  qr_swap<16>(y, b);
+  y = y + b;
+  b = y;
+  qr_swap<32>(y, b);
+  return y + b;
+}
+
+// |x|^2 of the panel's first column (in lane 0's result), whose sequences start with their second
+// row's rounded square, the first row's added by a multiply-add; the other rows in order.
+template <int NT>
+__device__ __attribute__((always_inline)) inline double qo_first_norm2(const qo_acc_t (&acc)[NT], int P) {
+  qo_acc_t s[4], h[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) s[i] = h[i] = qo_acc_t{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    if (t < P) continue;
+    qo_acc_t& st = s[t & 3];
+    const qo_acc_t x = acc[t];
+    if (t < P + 4) h[t & 3] = x;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      if (t >= P + 8) st[v] = fma(x[v], x[v], st[v]);
+      else if (t >= P + 4) st[v] = fma(h[t & 3][v], h[t & 3][v], x[v] * x[v]);
+      else st[v] = x[v] * x[v];
+    }
+  }
+  return qo_combine<NT>(s);
+}
+
+// Householder steps of columns 4 HV .. 4 HV + 3 (below w) of panel P, the strip kept in the
+// accumulator layout: lane l holds column l % 16, rows l / 16 + 4 v of each tile.  The pivot column
+// goes through LDS (xbuf) to the other columns' lanes, which need the same rows: the products x^T
+// col of every column are then one multiply-add per element and a sum over four lanes, and the
+// update is another multiply-add.  With beta = -sign(alpha) |x|, tau = (beta - alpha) / beta and
+// v = x / (alpha - beta) (row j: 1), col -= v (tau v^T col); a column of V stays x's tail, unscaled,
+// until the panel is done, and row j of R goes to rbuf.
+// The summation order is fixed (a rounding of the recompute grows by orders of magnitude in the
+// wraps that follow it): row 16 P + p of the panel belongs to sequence p % 64, which sums its rows
+// in order (the first column's norm: qo_first_norm2), and qo_combine adds the sequences.
+// Bound by the dependent chain of a column (LDS round trip, sums, root and divisions) and its
+// issue, not by its flops: the row-in-tile HV is a constant, and up to 8 tiles are worked on
+// without branches.
+template <int NT, int HV>
+__device__ __attribute__((always_inline)) inline void qo_columns(qo_acc_t (&acc)[NT], QoPanel& p, const QoShared& sh,
+                                                                 int P, int w, const int (&xo)[NT], double xx0) {
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+  qo_acc_t* xw = reinterpret_cast<qo_acc_t*>(sh.xbuf) + lk;  // [tile][l / 16]
+#pragma unroll 1
+  for (int hk = 0; hk < 4; ++hk) {
+    const int q = 4 * HV + hk;
+    if (q >= w) break;
+    qr_wave_sync();  // the previous column's reads are done
+    if (li == q) {
+#pragma unroll
+      for (int t = 1; t < NT; ++t) xw[xo[t]] = acc[t];
+      qo_acc_t m;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) m[v] = v < HV ? 0.0 : (v > HV || lk >= hk ? p.pt[v] : 0.0);
+      xw[4 * P] = m;
+    }
+    qr_wave_sync();
+    qo_acc_t x[NT];
+    if constexpr (NT <= 8) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) x[t] = xw[4 * t];
+    }
+    // row j of every column (the other three terms are zeros)
+    double bc = lk == hk ? p.pt[HV] : 0.0;
+    {
+      double b2 = bc;
+      qr_swap<16>(bc, b2);
+      bc = bc + b2;
+      b2 = bc;
+      qr_swap<32>(bc, b2);
+      bc = bc + b2;
+    }
+    const double alpha = qo_readlane(bc, q);
+    // x^T col over rows >= j
+    qo_acc_t s[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s[i] = qo_acc_t{0.0, 0.0, 0.0, 0.0};
+    qo_tiles<NT>(xw, x, P, [&](int t, const qo_acc_t& xt) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) s[t & 3][v] = fma(xt[v], acc[t][v], s[t & 3][v]);
+    });
+    const double y = qo_combine<NT>(s);
+    const double xx = NT > 4 && HV == 0 && hk == 0 ? xx0 : qo_readlane(y, q);
+    double nrm = qo_sqrt(xx);
+    double beta = alpha >= 0.0 ? -nrm : nrm;
+    double tau = qo_div(beta - alpha, beta), scal = qo_div(1.0, alpha - beta);
+    if (__builtin_expect(!(xx > 1e-200 && xx < 1e200), 0)) {
+      nrm = sqrt(xx > 0.0 ? xx : 0.0);
+      if (nrm == 0.0) {
+        beta = tau = scal = 0.0;
+        p.zero = true;
       } else {
-        beta = alpha >= 0.0 ? -nrmv : nrmv;
+        beta = alpha >= 0.0 ? -nrm : nrm;
         tau = (beta - alpha) / beta;
         scal = 1.0 / (alpha - beta);
       }
-      const double ts = tau * scal;
-      double v[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int r = j0 + lane + 64 * i;
-        v[i] = r > j ? x[i][q] * scal : (r == j ? 1.0 : 0.0);
-      }
-      // column c -= v (tau v^T col_c), tau v^T col_c = ts (s_c - beta col_c[j]), v = u / (alpha - beta)
-#pragma unroll
-      for (int c = q + 1; c < 16; ++c) {
-        const double dpc = c < w ? ts * (sh.red[c] - beta * qo_readlane(x[0][c], q)) : 0.0;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) x[i][c] = x[i][c] - v[i] * dpc;
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int r = j0 + lane + 64 * i;
-        x[i][q] = r > j ? v[i] : (r == j ? beta : x[i][q]);
-      }
-      qr_wave_sync();  // red read by every lane before the next reduction writes it
-      if (lane == 0) {
-        sh.taus[q] = tau;
-        const double d = fabs(beta);
-        sh.dbuf[j] = d > 0.0 ? d : 1e-300;
-      }
     }
-  }
-  // V (explicit) to vbuf, reflectors to A, R to sbuf
+    const double dpc = li > q ? (tau * scal) * fma(-beta, bc, y) : 0.0;
+    {
+      const qo_acc_t xd = xw[4 * P];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = j0 + lane + 64 * i;
-    if (r >= QO_NMAX) continue;
-    const bool in = r < N;
-#pragma unroll
-    for (int c = 0; c < 16; ++c) {
-      const int jc = j0 + c;
-      const bool col = c < w;
-      sh.vbuf[r * QO_PS + c] = (in && col) ? (r > jc ? x[i][c] : (r == jc ? 1.0 : 0.0)) : 0.0;
-      if (in && col && r <= jc) sbuf[r * QO_PS + c] = x[i][c];
-      if (in && col && r > jc) tk.A[(size_t)r * N + jc] = x[i][c];
+      for (int v = HV; v < 4; ++v) p.pt[v] = fma(-(xd[v] * scal), dpc, p.pt[v]);
     }
+    qo_tiles<NT>(xw, x, P, [&](int t, const qo_acc_t& xt) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) acc[t][v] = fma(-(xt[v] * scal), dpc, acc[t][v]);
+    });
+    if (lk == 0) sh.rbuf[q * 16 + li] = li == q ? beta : bc - dpc;  // row j of R (columns >= q)
+    if (lane == 0) sh.taus[q] = tau;
+    p.scal = li == q ? scal : p.scal;
+    p.beta = li == q ? beta : p.beta;
   }
+}
+
+// Panel P (w columns) of the calling wavefront's strip: V (explicit) to the LDS buffer of the
+// panel's parity, |diag R| to dbuf.  On return the strip's registers hold R on and above the
+// diagonal and V below it (columns past w are zero).
+template <int NT>
+__device__ __attribute__((always_inline)) inline void qo_factor(qo_acc_t (&acc)[NT], const QoShared& sh, int NS, int P,
+                                                                int w, bool& zero_pivot) {
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+  QoPanel p;
+  p.scal = 0.0;
+  p.beta = 0.0;
+  p.zero = false;
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    double e = acc[0][v];
+#pragma unroll
+    for (int t = 1; t < NT; ++t) {
+      const double a = acc[t][v];
+      e = t == P ? a : e;
+    }
+    p.pt[v] = e;
+  }
+  // tiles before P take no part: their x is zero, and writes of it go to an unread slot
+  int xo[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    xo[t] = t > P ? 4 * t : 4 * NT;
+    if (li == 0 && t < P) reinterpret_cast<qo_acc_t*>(sh.xbuf)[4 * t + lk] = qo_acc_t{0.0, 0.0, 0.0, 0.0};
+  }
+  const double xx0 = NT > 4 ? qo_readlane(qo_first_norm2<NT>(acc, P), 0) : 0.0;
+  qo_columns<NT, 0>(acc, p, sh, P, w, xo, xx0);
+  qo_columns<NT, 1>(acc, p, sh, P, w, xo, 0.0);
+  qo_columns<NT, 2>(acc, p, sh, P, w, xo, 0.0);
+  qo_columns<NT, 3>(acc, p, sh, P, w, xo, 0.0);
+  if (p.zero) zero_pivot = true;
+  double* vb = sh.vbuf + (P & 1) * sh.vs;
   qr_wave_sync();
-  qr_build_t(sh.vbuf, QO_PS, 16, j0, N, w, sh.taus, sh.tbuf, sh.ssc);
-  double* tout = tk.Tt + (size_t)P * 256;
-  for (int e = lane; e < 256; e += 64) tout[e] = ((e >> 4) < w && (e & 15) < w) ? sh.tbuf[e] : 0.0;
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    const int r = lk + 4 * v;
+    const double rv = ld0(sh.rbuf, (size_t)(r * 16 + li), r <= li && r < w);
+    p.pt[v] = r > li ? p.pt[v] * p.scal : rv;
+    vb[(16 * P + r) * QO_PS + li] = r > li ? p.pt[v] : (r == li && li < w ? 1.0 : 0.0);
+  }
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    if (t <= P || t >= NS) continue;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      acc[t][v] = acc[t][v] * p.scal;
+      vb[(16 * t + lk + 4 * v) * QO_PS + li] = acc[t][v];
+    }
+  }
+  if (lk == 0 && li < w) {
+    const double d = fabs(p.beta);
+    sh.dbuf[16 * P + li] = d > 0.0 ? d : 1e-300;
+  }
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const double a = acc[t][v], b = p.pt[v];
+      acc[t][v] = t == P ? b : a;
+    }
+}
+
+// T of panel P from the V left in the strip's registers: S = V^T V on the matrix cores (the
+// accumulator layout is the operand layout), then column by column T[:, i] = -tau_i T S[:, i], the
+// terms of a sum in order.  Runs on the panel's wavefront while the others form V^T X.
+template <int NT>
+__device__ __attribute__((always_inline)) inline void qo_form_t(const qo_acc_t (&acc)[NT], const QoShared& sh, int NS,
+                                                                int P, int w) {
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+  qr_v4d sa = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    if (t < P || t >= NS) continue;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int r = lk + 4 * v;
+      double e = acc[t][v];
+      if (t == P) e = r > li ? e : (r == li && li < w ? 1.0 : 0.0);
+      sa = qr_mma(e, e, sa);
+    }
+  }
+#pragma unroll
+  for (int v = 0; v < 4; ++v) sh.ssc[(lk + 4 * v) * 16 + li] = sa[v];
+  qr_wave_sync();
+  double* tb = sh.tbuf + (P & 1) * 256;
+  // lane p = li forms row p: sum[i] collects T[p][q] S[q][i] as the T[p][q] become final
+  double sum[16], tr[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) sum[i] = 0.0;
+#pragma unroll
+  for (int q = 0; q < 16; ++q) {
+    const double tq = sh.taus[q];
+    double t = q < li ? 0.0 : (q == li ? tq : -tq * sum[q]);
+    if (q >= w || li >= w) t = 0.0;
+    tr[q] = t;
+#pragma unroll
+    for (int i = q + 1; i < 16; ++i) {
+      const double e = fma(t, sh.ssc[q * 16 + i], sum[i]);
+      sum[i] = q >= li ? e : sum[i];
+    }
+  }
+  if (lk == 0)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) tb[li * 16 + i] = tr[i];
+}
+
+// After panel P is released to the other wavefronts, off the panel chain: its reflectors (below
+// the diagonal of A), T and |diag R| to memory, for the right half of a split matrix and for Q
+// formation, and the strip's columns of D^-1 R over W: V'' = D^-1 R P^T (columns to their original
+// places), or R' = D^-1 R with the pivot order.  hand: the matrix's hand-over counters in the left
+// half of a split matrix, else null.
+template <int NT>
+__device__ __attribute__((always_inline)) inline void qo_publish(const qo_acc_t (&acc)[NT], const QrTask& tk,
+                                                                 const QoShared& sh, const int* perm, int N, int P,
+                                                                 int w, unsigned* hand, ChainState* st, bool& broken) {
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+  const int j0 = P << 4, jc = j0 + li;
+  const double* tb = sh.tbuf + (P & 1) * 256;
+  LQMC_GLOBAL double* tout = gptr(tk.Tt) + P * 256;
+  for (int e = lane; e < 256; e += 64) tout[e] = tb[e];
   if (lane < w) tk.D[j0 + lane] = sh.dbuf[j0 + lane];
-  if (hand && left) {
-    // hand the panel (reflectors in A, T in Tt, D) to the right half
+  {
+    LQMC_GLOBAL double* A = gptr(tk.A);
+    const int vo = lk * N + jc;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      if (t < P || 16 * t >= N) continue;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int r = 16 * t + lk + 4 * v;
+        if (r < N && li < w && r > jc) (A + (16 * t + 4 * v) * N)[vo] = acc[t][v];
+      }
+    }
+  }
+  if (hand) {
     __builtin_amdgcn_s_waitcnt(0);
     qr_wave_sync();
     if (lane == 0) {
@@ -1017,22 +1274,176 @@ __device__ void qo_factor(qo_acc_t (&acc)[16], const QrTask& tk, const QoShared&
     }
     qr_wave_sync();
   }
+  if (li < w) {
+    LQMC_GLOBAL double* W = gptr(tk.W);
+    const int vo = lk * N + (tk.perm ? jc : perm[jc]);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      if (16 * t >= N) continue;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int r = 16 * t + lk + 4 * v;
+        double e = 0.0;
+        if (t <= P && r <= jc) e = acc[t][v] / sh.dbuf[r];
+        if (r < N) (W + (16 * t + 4 * v) * N)[vo] = e;
+      }
+    }
+  }
 }
 
-// R of strip S (rows 0..16S+15, upper triangle of the panel block) from sbuf back to the
-// accumulator layout; zero below.  Runs after the panel's release barrier, while the next
-// wavefront applies the panel and before it overwrites sbuf.
-__device__ inline void qo_keep_r(qo_acc_t (&acc)[16], const QoShared& sh, int S) {
-  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
-  const int jc = 16 * S + li;
+// The factorisation with NT >= NS row tiles per strip, one wavefront per strip of the workgroup's
+// half (SPLIT) or of the matrix; perm: the pre-pivot order.
+template <int NT, bool SPLIT>
+__device__ __attribute__((always_inline)) inline void qo_run(const QrTask& tk, const QoShared& sh, const int* perm,
+                                                             int part, unsigned* hd, ChainState* st, bool& zero_pivot,
+                                                             bool& broken) {
+  const int N = tk.N;
+  const int NS = (N + 15) >> 4;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int li = lane & 15, lk = lane >> 4;
+  // my strip (wavefront-uniform, in a scalar register)
+  const int S = part * 8 + __builtin_amdgcn_readlane(tid >> 6, 0);
+  const bool have = S < NS;
+  qo_acc_t acc[NT];
+  {
+    const int c = 16 * S + li;
+    const bool cok = have && c < N;
+    const int vo = lk * N + perm[cok ? c : 0];
 #pragma unroll
-  for (int t = 0; t < 16; ++t)
+    for (int t = 0; t < NT; ++t)
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int r = 16 * t + lk + 4 * v;
-      acc[t][v] = ld0(sh.sbuf, (size_t)r * QO_PS + li, r <= jc);
+      for (int v = 0; v < 4; ++v) {
+        const int r = 16 * t + lk + 4 * v;
+        acc[t][v] = ldg0(gptr(tk.W), (size_t)((16 * t + 4 * v) * N + vo), cok && r < N);
+      }
+  }
+  // every read of W is complete before any workgroup of the matrix writes it
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  const int P0 = SPLIT ? part * 8 : 0, P1 = SPLIT ? min(NS, P0 + 8) : NS;  // the panels of my half
+  if constexpr (SPLIT) {
+    if (part == 1 && tid == 0) {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+      atomicExch(hd + 1, 1u);
     }
+    // 1. panels received from the left half
+#pragma unroll 1
+    for (int P = 0; P < P0; ++P) {
+      const int j0 = P << 4, w = min(16, N - j0);
+      if (tid == 0) qo_wait(hd, (unsigned)P, st, tk.chain, broken);
+      __syncthreads();
+      double* vb = sh.vbuf + (P & 1) * sh.vs;
+      for (int e = tid; e < (QO_NMAX - j0) * 16; e += QO_THREADS) {
+        const int r = j0 + (e >> 4), c = e & 15, jc = j0 + c;
+        const bool in = r < N && c < w;
+        const double a = ldg0(gptr(tk.A), (size_t)r * N + jc, in && r > jc);
+        vb[r * QO_PS + c] = in ? (r > jc ? a : (r == jc ? 1.0 : 0.0)) : 0.0;
+      }
+      for (int e = tid; e < 256; e += QO_THREADS) sh.tbuf[(P & 1) * 256 + e] = tk.Tt[(size_t)P * 256 + e];
+      if (tid < w) sh.dbuf[j0 + tid] = tk.D[j0 + tid];
+      __syncthreads();
+      if (have) qo_apply<NT>(acc, vb, sh.tbuf + (P & 1) * 256, NS, P);
+    }
+  }
+  // 2. my half's panels, two barriers each: V is there, T is there.  The buffers of a panel's
+  //    parity are free when its wavefront writes them: every wavefront applied panel P - 2
+  //    before the barriers of P - 1.
+  const int Sm = have ? S : P1;
+#pragma unroll 1
+  for (int P = P0; P < Sm; ++P) {
+    const double* vb = sh.vbuf + (P & 1) * sh.vs;
+    __syncthreads();
+    qr_v4d wt = {0.0, 0.0, 0.0, 0.0};
+    if (have) {
+      if (P + 1 == S) LQMC_WAVE_PRIO(3);  // the next panel waits for this strip
+      wt = qo_apply_vt<NT>(acc, vb, NS, P);
+    }
+    __syncthreads();
+    if (have) qo_apply_v<NT>(acc, vb, sh.tbuf + (P & 1) * 256, wt, NS, P);
+  }
+  if (have) {
+    const int w = min(16, N - 16 * S);
+    LQMC_WAVE_PRIO(3);
+    qo_factor<NT>(acc, sh, NS, S, w, zero_pivot);
+    __syncthreads();
+    qo_form_t<NT>(acc, sh, NS, S, w);
+    LQMC_WAVE_PRIO(0);
+    __syncthreads();
+    qo_publish<NT>(acc, tk, sh, perm, N, S, w, SPLIT && part == 0 ? hd : nullptr, st, broken);
+#pragma unroll 1
+    for (int P = S + 1; P < P1; ++P) {
+      __syncthreads();
+      __syncthreads();
+    }
+  }
+  if constexpr (SPLIT) {
+    __syncthreads();
+    if (tid == 0) atomicExch(hd + (part == 1 ? 0 : 1), 0u);  // counters back to zero for the next launch
+  }
 }
+
+// Pre-pivoting: column norms (partial sums over TH / N row groups, combined in group order, so
+// that both workgroups of a split matrix, and workgroups of any size, derive the same order),
+// then decreasing norm, ties by index, NaN last.  scr: TH scratch, norms [N], perm [N]; dbuf
+// set to 1.
+template <int TH>
+__device__ inline bool qo_prepivot(const QrTask& tk, double* scr, double* norms, int* perm, double* dbuf) {
+  const int N = tk.N, tid = threadIdx.x, nth = blockDim.x;
+  bool bad = false;
+  const int ng = TH / N;  // >= 2 row groups
+  for (int e = tid; e < ng * N; e += nth) {
+    const int c = e % N, g = e / N;
+    double s = 0.0;
+    for (int r0 = g; r0 < N; r0 += 8 * ng) {
+      double xv[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int r = r0 + u * ng;
+        xv[u] = ldg0(gptr(tk.W), (size_t)r * N + c, r < N);
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u) s += xv[u] * xv[u];
+    }
+    scr[g * N + c] = s;
+  }
+  __syncthreads();
+  for (int c = tid; c < N; c += nth) {
+    double s = 0.0;
+    for (int g = 0; g < ng; ++g) s += scr[g * N + c];
+    if (!(s >= 0.0)) { s = -1.0; bad = true; }
+    norms[c] = s;
+  }
+  for (int i = tid; i < N; i += nth) dbuf[i] = 1.0;
+  __syncthreads();
+  for (int c = tid; c < N; c += nth) {
+    const double nc = norms[c];
+    int rank = 0;
+#pragma unroll 8
+    for (int c2 = 0; c2 < N; ++c2) {
+      const double n2 = norms[c2];
+      rank += (n2 > nc) || (n2 == nc && c2 < c);
+    }
+    perm[rank] = c;
+  }
+  __syncthreads();
+  return bad;
+}
+
+// ROWS: rows that V is kept for.
+template <int ROWS>
+__device__ inline QoShared qo_shared(double* sm) {
+  QoShared sh;
+  sh.vs = ROWS * QO_PS;
+  sh.vbuf = sm;
+  sh.tbuf = sh.vbuf + 2 * ROWS * QO_PS;
+  sh.xbuf = sh.tbuf + 512;
+  sh.rbuf = sh.xbuf + ROWS + 16;
+  sh.ssc = sh.rbuf + 256;
+  sh.taus = sh.ssc + 256;
+  sh.dbuf = sh.taus + 16;
+  return sh;
+}
+constexpr int qo_lds(int rows) { return 2 * rows * QO_PS + 512 + rows + 16 + 256 + 256 + 16 + rows; }  // doubles
 
 __global__ __launch_bounds__(QO_THREADS) void k_qr_onchip(const QrTask* __restrict__ tasks, int ntasks, int G,
                                                           unsigned* hand, ChainState* st) {
@@ -1041,157 +1452,50 @@ __global__ __launch_bounds__(QO_THREADS) void k_qr_onchip(const QrTask* __restri
   if (ti >= ntasks) return;
   const QrTask tk = tasks[ti];
   const int N = tk.N;
-  const int NS = (N + 15) >> 4;   // strips, and row tiles
   const int Gt = (N + 127) >> 7;  // workgroups this matrix uses
   if (part >= Gt) return;
-  unsigned* hd = Gt > 1 ? hand + 2 * ti : nullptr;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int li = lane & 15, lk = lane >> 4;
+  const int tid = threadIdx.x, lane = tid & 63;
   LQMC_DYNAMIC_LDS(double, sm);
-  QoShared sh;
-  sh.sbuf = sm;                             // [256][17] strip transpose buffer, pre-pivot partials
-  sh.vbuf = sh.sbuf + QO_NMAX * QO_PS;      // [256][17] explicit V of the current panel
-  sh.tbuf = sh.vbuf + QO_NMAX * QO_PS;      // [16][16] T of the current panel
-  sh.ssc = sh.tbuf + 256;                   // [16][16] S = V^T V scratch
-  sh.red = sh.ssc + 256;                    // [16] wavefront column sums
-  sh.dbuf = sh.red + 16;                    // [256] |diag R|
-  sh.taus = sh.dbuf + QO_NMAX;              // [16] reflector coefficients of the panel
-  double* norms = sh.taus + 16;             // [256] pre-pivot column norms
+  double* norms = sm;                                   // [256] pre-pivot column norms
   int* perm = reinterpret_cast<int*>(norms + QO_NMAX);  // [256] pre-pivot order
-  sh.perm = perm;
-  bool zero_pivot = false, bad = false, broken = false;
-
-  // pre-pivoting: column norms (partial sums over row groups, combined in group order, so
-  // both workgroups of a matrix derive the same order), then decreasing norm, ties by index,
-  // NaN last
-  {
-    const int ng = QO_THREADS / N;  // >= 2 row groups
-    if (tid < ng * N) {
-      const int c = tid % N, g = tid / N;
-      double s = 0.0;
-      for (int r0 = g; r0 < N; r0 += 8 * ng) {
-        double xv[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          const int r = r0 + u * ng;
-          xv[u] = ldg0(gptr(tk.W), (size_t)r * N + c, r < N);
-        }
-#pragma unroll
-        for (int u = 0; u < 8; ++u) s += xv[u] * xv[u];
-      }
-      sh.sbuf[g * N + c] = s;
-    }
-    __syncthreads();
-    for (int c = tid; c < N; c += QO_THREADS) {
-      double s = 0.0;
-      for (int g = 0; g < ng; ++g) s += sh.sbuf[g * N + c];
-      if (!(s >= 0.0)) { s = -1.0; bad = true; }
-      norms[c] = s;
-    }
-    for (int i = tid; i < QO_NMAX; i += QO_THREADS) sh.dbuf[i] = 1.0;
-    __syncthreads();
-    for (int c = tid; c < N; c += QO_THREADS) {
-      const double nc = norms[c];
-      int rank = 0;
-      for (int c2 = 0; c2 < N; ++c2) {
-        const double n2 = norms[c2];
-        rank += (n2 > nc) || (n2 == nc && c2 < c);
-      }
-      perm[rank] = c;
-    }
-    __syncthreads();
-  }
-  // my strip
-  const int S = part * 8 + wave;
-  const bool have = S < NS;
-  qo_acc_t acc[16];
-  {
-    const int c = 16 * S + li;
-    const bool cok = have && c < N;
-    const int pc = perm[cok ? c : 0];
-#pragma unroll
-    for (int t = 0; t < 16; ++t)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int r = 16 * t + lk + 4 * v;
-        acc[t][v] = ldg0(gptr(tk.W), (size_t)r * N + pc, cok && r < N);
-      }
-  }
-  // every read of W is complete before any workgroup of the matrix writes it
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
-  if (hd && part == 1 && tid == 0) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    atomicExch(hd + 1, 1u);
-  }
-  const int P0 = part * 8, P1 = min(NS, P0 + 8);  // the panels of my half
-  const int Sm = have ? S : P1;
-  // 1. panels left of my strip (received from the left half, or factored by a wavefront of
-  //    my half before the first barrier of their iteration)
-  for (int P = 0; P < Sm; ++P) {
-    if (P < P0) {
-      const int j0 = P << 4, w = min(16, N - j0);
-      if (tid == 0) qo_wait(hd, (unsigned)P, st, tk.chain, broken);
-      __syncthreads();
-      for (int e = tid; e < (QO_NMAX - j0) * 16; e += QO_THREADS) {
-        const int r = j0 + (e >> 4), c = e & 15, jc = j0 + c;
-        const bool in = r < N && c < w;
-        const double a = ldg0(gptr(tk.A), (size_t)r * N + jc, in && r > jc);
-        sh.vbuf[r * QO_PS + c] = in ? (r > jc ? a : (r == jc ? 1.0 : 0.0)) : 0.0;
-      }
-      for (int e = tid; e < 256; e += QO_THREADS) sh.tbuf[e] = tk.Tt[(size_t)P * 256 + e];
-      if (tid < w) sh.dbuf[j0 + tid] = tk.D[j0 + tid];
-    }
-    __syncthreads();
-    if (have) qo_apply(acc, sh.vbuf, sh.tbuf, NS, P);
-    __syncthreads();
-  }
-  // 2. my panel, 3. the panels right of it
-  if (have) {
-    qo_factor(acc, tk, sh, N, S, min(16, N - 16 * S), hd, part == 0, st, broken, zero_pivot);
-    __syncthreads();
-    qo_keep_r(acc, sh, S);
-    __syncthreads();
-    for (int P = S + 1; P < P1; ++P) {
-      __syncthreads();
-      __syncthreads();
-    }
-  }
-  __syncthreads();
-  if (hd && tid == 0) atomicExch(hd + (part == 1 ? 0 : 1), 0u);  // counters back to zero for the next launch
+  const QoShared sh = qo_shared<QO_NMAX>(norms + QO_NMAX + QO_NMAX / 2);
+  bool zero_pivot = false, broken = false;
+  const bool bad = qo_prepivot<QO_THREADS>(tk, sh.vbuf, norms, perm, sh.dbuf);
   if (part == 0 && tk.perm)
     for (int i = tid; i < N; i += QO_THREADS) tk.perm[i] = perm[i];
-  // 4. D^-1 R of my strip over W: V'' = D^-1 R P^T (columns to their original places), or
-  //    R' = D^-1 R with the pivot order.  Off the panel chain: every |diag R| this strip
-  //    needs (rows <= its last column) is in dbuf by now.
-  if (have) {
-    // N and the lane's row made opaque, so the compiler forms these 64 row offsets and
-    // bounds here instead of keeping those of the strip load live all kernel (128 VGPRs)
-    int Nw = N, lkw = lk;
-    LQMC_OPAQUE(Nw, "s");
-    LQMC_OPAQUE(lkw, "v");
-    const int jc = 16 * S + li;
-    if (jc < Nw) {
-      const int oc = tk.perm ? jc : perm[jc];
-#pragma unroll
-      for (int t = 0; t < 16; ++t)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int r = 16 * t + lkw + 4 * v;
-          if (r < Nw) tk.W[(size_t)r * Nw + oc] = r <= jc ? acc[t][v] / sh.dbuf[r] : 0.0;
-        }
-    }
-  }
+  if (Gt > 1) qo_run<16, true>(tk, sh, perm, part, hand + 2 * ti, st, zero_pivot, broken);
+  else qo_run<8, false>(tk, sh, perm, 0, nullptr, st, zero_pivot, broken);
   if (st) {
     if (zero_pivot && lane == 0) atomicOr(&st[tk.chain].flags, 2u);
     if (bad) atomicOr(&st[tk.chain].flags, 8u);
   }
 }
 
-size_t qr_onchip_shmem() {
-  return sizeof(double) * (2 * (size_t)QO_NMAX * QO_PS + 256 + 256 + 16 + QO_NMAX + 16 + QO_NMAX) +
-         sizeof(int) * QO_NMAX;
+// N <= 64: the same factorisation by four wavefronts holding 16 x 64 strips, so that several
+// matrices share a compute unit.
+constexpr int QU_THREADS = 256;
+__global__ __launch_bounds__(QU_THREADS, 2) void k_qr_small(const QrTask* __restrict__ tasks, ChainState* st) {
+  const QrTask tk = tasks[blockIdx.x];
+  const int N = tk.N, tid = threadIdx.x;
+  LQMC_DYNAMIC_LDS(double, sm);
+  double* norms = sm;                              // [64] pre-pivot column norms
+  int* perm = reinterpret_cast<int*>(norms + 64);  // [64] pre-pivot order
+  const QoShared sh = qo_shared<64>(norms + 96);
+  bool zero_pivot = false, broken = false;
+  // (the scratch of the norms, 512 doubles, lies in vbuf)
+  const bool bad = qo_prepivot<QO_THREADS>(tk, sh.vbuf, norms, perm, sh.dbuf);
+  if (tk.perm)
+    for (int i = tid; i < N; i += QU_THREADS) tk.perm[i] = perm[i];
+  if (N <= 32) qo_run<2, false>(tk, sh, perm, 0, nullptr, st, zero_pivot, broken);
+  else qo_run<4, false>(tk, sh, perm, 0, nullptr, st, zero_pivot, broken);
+  if (st) {
+    if (zero_pivot && (tid & 63) == 0) atomicOr(&st[tk.chain].flags, 2u);
+    if (bad) atomicOr(&st[tk.chain].flags, 8u);
+  }
 }
+size_t qr_small_shmem() { return sizeof(double) * (96 + qo_lds(64)); }
+
+size_t qr_onchip_shmem() { return sizeof(double) * (QO_NMAX + QO_NMAX / 2 + (size_t)qo_lds(QO_NMAX)); }
 
 size_t qr_blocked_shmem(int nmax) {
   const size_t nb = nmax > 256 ? 8 : 16;
@@ -1211,7 +1515,9 @@ size_t trsm_shmem(int) { return sizeof(double) * (TRSM_B * QF_COLS + TRSM_B * TR
 // larger N: the blocked factorisation with the trailing matrix in global memory.
 void launch_qr_blocked(const QrTask* d, int n, int nmax, ChainState* st, unsigned* hand, int max_wg, hipStream_t s) {
   if (n <= 0) return;
-  if (nmax <= QO_NMAX) {
+  if (nmax <= 64) {
+    hipLaunchKernelGGL(k_qr_small, dim3(n), dim3(QU_THREADS), qr_small_shmem(), s, d, st);
+  } else if (nmax <= QO_NMAX) {
     static bool attr = false;
     if (!attr) {
       (void)hipFuncSetAttribute((const void*)k_qr_onchip, hipFuncAttributeMaxDynamicSharedMemorySize,
