@@ -203,6 +203,7 @@ struct FlipArgs {
   int bf3;        // delayed FP32 form: rank-k products as three split-BF16 matrix-core products
   int yrows;      // delayed flip, k = 16, one spin per workgroup: the block's rows of G and its Z tiles
                   // kept in LDS (flip_delayed_stage_rows; flip_delayed_rows_shmem more bytes of LDS)
+  const int* list;  // the launch's nchains chains (null: chains 0 .. nchains-1)
 };
 
 }  // namespace lqmc

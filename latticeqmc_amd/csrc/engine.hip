@@ -42,6 +42,8 @@ void launch_green_out(double* out, const void* src, int fp32, size_t n, const Ch
                       hipStream_t s);
 void launch_flip(int fp32, int delayed, const FlipArgs& a, int nchains, int threads, size_t shmem,
                  hipStream_t s);
+void launch_flip_tile(int cls, const FlipArgs& a, hipStream_t s);
+int flip_tile_class(int N);
 size_t flip_delayed_shmem(int nmax, int k, int threads, int fp32);
 size_t flip_delayed_workspace(int n, int k, int fp32, int groups);
 int flip_delayed_stage_rows(int nmax, int k, int groups);
@@ -158,6 +160,11 @@ struct lqmc_ctx {
   double** d_eye_ptrs = nullptr;
   int* d_eye_ns = nullptr;
   int nmax = 0, lmax = 0;
+  // flips: chains [tile_off[k], tile_off[k+1]) of the list in the register-tile form of class k, the
+  // others (from tile_off[8] on) in the form that the options name
+  int* d_flip_list = nullptr;
+  int tile_off[9] = {};
+  int flip_rest = 0;             // chains from tile_off[8] on
   int flip_threads = 256;
   int flip_groups = 1;           // workgroups per chain of the delayed flip
   int flip_yrows = 0;            // delayed flip keeps block rows and Z tiles in LDS (FlipArgs::yrows)
@@ -721,8 +728,17 @@ static void run_ops(lqmc_ctx* x, const std::vector<Op>& ops, int measure, hipStr
       case OP_FLIP: {
         FlipArgs a{x->d_chains, x->d_state, op.t, measure, x->opt.rng, x->opt.trace, x->opt.delay,
                    x->flip_groups, x->d_bar, x->nchains, x->opt.precision == LQMC_BF16X3 ? 1 : 0,
-                   x->flip_yrows};
-        launch_flip(fp32, x->opt.delay > 1, a, x->nchains, x->flip_threads, x->flip_shmem, s);
+                   x->flip_yrows, nullptr};
+        for (int k = 0; k < 8; ++k) {
+          a.nchains = x->tile_off[k + 1] - x->tile_off[k];
+          a.list = x->d_flip_list + x->tile_off[k];
+          launch_flip_tile(k, a, s);
+        }
+        if (x->flip_rest) {
+          a.nchains = x->flip_rest;
+          a.list = x->d_flip_list + x->tile_off[8];
+          launch_flip(fp32, x->opt.delay > 1, a, x->flip_rest, x->flip_threads, x->flip_shmem, s);
+        }
         break;
       }
     }
@@ -790,6 +806,12 @@ int lqmc_create(lqmc_ctx** out, int device, int n_chains, const int32_t* n_sites
     x->nmax = std::max(x->nmax, (int)n_sites[c]);
     x->lmax = std::max(x->lmax, (int)time_steps[c]);
   }
+  // FP64 Mode D chains of up to 128 sites flip in registers (flip_tile.hip) unless the options name a
+  // form of the other flip kernels; nrest / nmax_rest: the chains left to those.
+  const bool tiled = o.mode == LQMC_MODE_DQMC && o.precision == LQMC_FP64 && o.flip_threads == 0 && o.flip_groups == 0;
+  int nrest = 0, nmax_rest = 0;
+  for (auto& c : x->ch)
+    if (!tiled || flip_tile_class(c.N) < 0) { ++nrest; nmax_rest = std::max(nmax_rest, c.N); }
   // The flip kernels keep their dynamic LDS within 64 KB per workgroup (the
   // delayed form's rank-k operands live in a per-chain global workspace), which
   // bounds the supported delay for a given thread count.  Only the delayed flip's
@@ -797,9 +819,10 @@ int lqmc_create(lqmc_ctx** out, int device, int n_chains, const int32_t* n_sites
   // device's per-workgroup LDS allows (160 KB on gfx950).
   const int maxsh = 65536;
   const bool fp32 = o.precision != LQMC_FP64;
+  const int nmax_flip = nrest ? nmax_rest : x->nmax;  // the size that the other flip kernels are set up for
   const int tmax = o.delay > 1 ? flip_delayed_threads_limit(o.delay) : 1024;
   if (o.flip_threads > 0) x->flip_threads = o.flip_threads;
-  else x->flip_threads = x->nmax >= 128 ? tmax : 256;
+  else x->flip_threads = nmax_flip >= 128 ? tmax : 256;
   const int tmin = o.delay > 1 ? 256 : 64;
   if (x->flip_threads % 64 || x->flip_threads > tmax || x->flip_threads < tmin) {
     char buf[128];
@@ -807,8 +830,8 @@ int lqmc_create(lqmc_ctx** out, int device, int n_chains, const int32_t* n_sites
     delete x;
     return fail(LQMC_EINVAL, buf);
   }
-  if (o.delay > 1) x->flip_shmem = flip_delayed_shmem(x->nmax, o.delay, x->flip_threads, fp32);
-  else x->flip_shmem = sizeof(double) * (4 * (size_t)x->nmax + x->flip_threads);
+  if (o.delay > 1) x->flip_shmem = flip_delayed_shmem(nmax_flip, o.delay, x->flip_threads, fp32);
+  else x->flip_shmem = sizeof(double) * (4 * (size_t)nmax_flip + x->flip_threads);
   if ((int)x->flip_shmem > maxsh) {
     char buf[160];
     snprintf(buf, sizeof buf, "flip kernel needs %zu B of LDS (> %d); lower the delay", x->flip_shmem, maxsh);
@@ -829,7 +852,8 @@ int lqmc_create(lqmc_ctx** out, int device, int n_chains, const int32_t* n_sites
     const int cus = prop.multiProcessorCount;
     x->cus = cus;
     lds_dev = prop.sharedMemPerBlock;
-    const int padded = 8 * ((n_chains + 7) / 8);
+    const int nflip = nrest ? nrest : n_chains;
+    const int padded = 8 * ((nflip + 7) / 8);
     const bool splittable = o.mode == LQMC_MODE_DQMC && (o.delay == 1 || o.delay == 16 || o.delay == 32);
     const int waves = x->flip_threads / 64;
     if (o.flip_groups < 0 || o.flip_groups > 64) {
@@ -850,15 +874,15 @@ int lqmc_create(lqmc_ctx** out, int device, int n_chains, const int32_t* n_sites
     if (o.flip_groups > 0) x->flip_groups = o.flip_groups;
     else if (splittable && o.delay > 1) {
       // at least one 16-row strip of either spin per wavefront
-      const int strips = 2 * ((x->nmax + 15) / 16);
+      const int strips = 2 * ((nmax_flip + 15) / 16);
       x->flip_groups = std::max(1, std::min(cus / padded, strips / waves));
     } else if (splittable) {
       // rank-1: at least 32 rows of each spin per workgroup
-      x->flip_groups = std::max(1, std::min(cus / padded, x->nmax / 32));
+      x->flip_groups = std::max(1, std::min(cus / padded, nmax_flip / 32));
     } else x->flip_groups = 1;
     if (o.delay == 1 && x->flip_groups > 1) {
       if (o.flip_threads <= 0) x->flip_threads = 512;
-      x->flip_shmem = flip_rank1_split_shmem(x->nmax, x->flip_threads, x->flip_groups);
+      x->flip_shmem = flip_rank1_split_shmem(nmax_flip, x->flip_threads, x->flip_groups);
       if ((int)x->flip_shmem > maxsh) {
         delete x;
         return fail(LQMC_EINVAL, "split rank-1 flip needs more than 64 KB of LDS");
@@ -866,10 +890,10 @@ int lqmc_create(lqmc_ctx** out, int device, int n_chains, const int32_t* n_sites
     }
   }
   // block rows and Z tiles of the delayed flip in LDS (k = 16, nmax <= 256), where they fit
-  if (o.delay > 1 && flip_delayed_stage_rows(x->nmax, o.delay, x->flip_groups) &&
-      x->flip_shmem + flip_delayed_rows_shmem(x->nmax, o.delay, x->flip_groups) <= lds_dev) {
+  if (o.delay > 1 && flip_delayed_stage_rows(nmax_flip, o.delay, x->flip_groups) &&
+      x->flip_shmem + flip_delayed_rows_shmem(nmax_flip, o.delay, x->flip_groups) <= lds_dev) {
     x->flip_yrows = 1;
-    x->flip_shmem += flip_delayed_rows_shmem(x->nmax, o.delay, x->flip_groups);
+    x->flip_shmem += flip_delayed_rows_shmem(nmax_flip, o.delay, x->flip_groups);
   }
   if (o.mode == LQMC_MODE_DET) {
     x->det_shmem = det_sweep_shmem(x->nmax, x->lmax);
@@ -911,6 +935,29 @@ int lqmc_create(lqmc_ctx** out, int device, int n_chains, const int32_t* n_sites
   off = 0;
   for (auto& c : x->ch) layout_chain(x, c, x->arena, off);
   x->h_chains.resize(n_chains);
+  {
+    // Flip launches: one per class present, or a single one in the largest class while every chain has
+    // a compute unit to itself (the launch then takes as long as its slowest chain either way).
+    std::vector<int> list, cls(n_chains, -1);
+    int top = -1;
+    for (int c = 0; c < n_chains; ++c)
+      if (tiled) { cls[c] = flip_tile_class(x->ch[c].N); top = std::max(top, cls[c]); }
+    const bool one = n_chains - nrest <= x->cus;
+    for (int k = 0; k < 8; ++k) {
+      x->tile_off[k] = (int)list.size();
+      for (int c = 0; c < n_chains; ++c)
+        if (cls[c] >= 0 && (one ? top : cls[c]) == k) list.push_back(c);
+    }
+    x->tile_off[8] = (int)list.size();
+    x->flip_rest = nrest;
+    for (int c = 0; c < n_chains; ++c)
+      if (cls[c] < 0) list.push_back(c);
+    if (hipMalloc(&x->d_flip_list, sizeof(int) * n_chains) != hipSuccess ||
+        hipMemcpy(x->d_flip_list, list.data(), sizeof(int) * n_chains, hipMemcpyHostToDevice) != hipSuccess) {
+      lqmc_destroy(x);
+      return fail(LQMC_ENOMEM, "flip list allocation failed");
+    }
+  }
   std::vector<double*> eyes(n_chains);
   std::vector<int> ns(n_chains);
   for (int c = 0; c < n_chains; ++c) { eyes[c] = x->ch[c].eye; ns[c] = x->ch[c].N; }
@@ -1371,6 +1418,7 @@ int lqmc_destroy(lqmc_ctx* x) {
   if (x->d_eye_ptrs) (void)hipFree(x->d_eye_ptrs);
   if (x->d_eye_ns) (void)hipFree(x->d_eye_ns);
   if (x->d_bar) (void)hipFree(x->d_bar);
+  if (x->d_flip_list) (void)hipFree(x->d_flip_list);
   if (x->d_qrpub) (void)hipFree(x->d_qrpub);
   if (x->done_ev) (void)hipEventDestroy(x->done_ev);
   if (x->aux_ev) (void)hipEventDestroy(x->aux_ev);
