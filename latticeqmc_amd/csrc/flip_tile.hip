@@ -12,12 +12,13 @@
 //   y = e_i - G[i, :], and on acceptance applies G -= x (c y)^T with T^2 multiply-adds.
 // The results do not depend on T and WR.
 //
-// Bound by the latency of the site chain (LDS round trip, barrier, ratio, division) and, from about
-// 64 sites on, by its T^2 multiply-adds; there are no block inverses, Z tiles or strip products, and
-// G crosses the memory system once per slice.  Per launch, against the delayed kernel that these
-// chains used before: 17.2 -> 8.2 us for one 4 x 4 chain, 69 -> 39 us for one 8 x 8 chain, 123 ->
-// 65 us for 8 chains of 84 sites, 318 -> 95 us for 256 chains of 36, 64 and 100 sites, 169 -> 119 us
-// for 32 chains of 117 sites.
+// Bound by the latency of the site chain (LDS round trip, barrier, ratio, division: about 900 cycles,
+// whatever T) and, from about 100 sites on, by the issue of its T^2 multiply-adds; there are no
+// block inverses, Z tiles or strip products, and G crosses the memory system once per slice.  The
+// uniforms and signs of eight sites are picked from registers, the parity of the buffers is a
+// constant and y's unit entry touches one register, which took a fifth off the chain.  Per launch,
+// against the delayed kernel that these chains used before: 17.2 -> 7.6 us for one 4 x 4 chain,
+// 69 -> 33 us for one 8 x 8 chain, 318 -> 82 us for 256 chains of 36, 64 and 100 sites.
 #include "flip_common.h"
 
 #include <algorithm>
@@ -39,6 +40,14 @@ __device__ inline double ft_div(double num, double d) {
 #endif
 }
 
+// Lane l's value (l wavefront-uniform) in scalar registers.
+__device__ inline double ft_readlane(double v, int l) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, l);
+  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b >> 32), l);
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
 template <int T, int WR>
 __global__ __launch_bounds__(128 * WR * WR) void k_flip_tile(FlipArgs a) {
   constexpr int NP = 8 * T * WR;  // sites covered
@@ -54,21 +63,20 @@ __global__ __launch_bounds__(128 * WR * WR) void k_flip_tile(FlipArgs a) {
   LQMC_DYNAMIC_LDS(double, sm);
   double* buf = sm;                // [2][PB]
   double* ub = buf + 2 * PB;       // [NP] uniforms
-  double* e2 = ub + NP;            // [NP] exp(2 lambda s) of the slice's sites
-  double* red = e2 + NP;           // blockDim (epilogue), and the trace of the slice before it
-  int8_t* acc_sh = reinterpret_cast<int8_t*>(red + std::max((int)blockDim.x, NP));  // [NP] accepted
+  double* red = ub + NP;           // blockDim (epilogue), and the slice's ratios before it (trace)
+  int* neg_sh = reinterpret_cast<int*>(red + std::max((int)blockDim.x, NP));  // [NP] spin is -1
+  int* acc_sh = neg_sh + NP;       // [NP / 8] accepted, a bit per site
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readlane(tid >> 6, 0);
   const int sp = wave / (WR * WR), wr = (wave / WR) % WR, wc = wave % WR;
   const int la = lane >> 3, lb = lane & 7;
   const int r0 = 8 * T * wr + la, c0 = 8 * T * wc + lb;  // my first row and column
-  bool underrun = false, bad = false;
+  bool underrun = false;
   {
     const unsigned long long sweep = a.st[c].sweep;
-    const double e2p = ch.e2p, e2m = ch.e2m;
-    for (int i = tid; i < N; i += blockDim.x) {
-      ub[i] = draw_uniform(ch, &a.st[c], c, a.rng, sweep, a.t, i, underrun);
-      e2[i] = fld[i] > 0 ? e2p : e2m;
+    for (int i = tid; i < NP; i += blockDim.x) {
+      ub[i] = i < N ? draw_uniform(ch, &a.st[c], c, a.rng, sweep, a.t, i, underrun) : 2.0;
+      neg_sh[i] = i < N && fld[i] < 0 ? 1 : 0;
     }
   }
   double g[T][T];
@@ -82,59 +90,67 @@ __global__ __launch_bounds__(128 * WR * WR) void k_flip_tile(FlipArgs a) {
         g[r][j] = ldg0(Gs, (size_t)row * N + col, row < N && col < N);
       }
   }
-  unsigned long long nacc = 0;
+  const double ap = ch.e2p - 1.0, am = ch.e2m - 1.0;  // alpha of a spin +1 (sigma = +1), and of a spin -1
+  double* const rowb = buf + sp * NP + c0;            // my part of row i of my spin
+  double* const colb = buf + (2 + sp) * NP + r0;      // my part of column i of my spin
+  unsigned nacc = 0;
+  double fin = 0.0;  // becomes NaN with the first ratio that is not finite
+  __syncthreads();
 #pragma unroll 1
   for (int q = 0; q < WR; ++q) {
 #pragma unroll
     for (int k = 0; k < T; ++k) {
+      const int i0 = 8 * (T * q + k);
+      if (i0 >= N) break;
+      // the uniforms and signs of these eight sites, site o in the lanes with lb = o
+      const double ul = ub[i0 + lb];
+      const int nl = neg_sh[i0 + lb];
+      unsigned abits = 0;
 #pragma unroll 1
-      for (int o = 0; o < 8; ++o) {
-        const int i = 8 * (T * q + k) + o;
-        if (i >= N) break;
-        double* pb = buf + (i & 1) * PB;
-        double* rowb = pb + sp * NP;           // row i of my spin
-        double* colb = pb + (2 + sp) * NP;     // column i of my spin
-        if (wr == q && la == o) {
+      for (int o2 = 0; o2 < 8; o2 += 2) {
 #pragma unroll
-          for (int j = 0; j < T; ++j) rowb[c0 + 8 * j] = g[k][j];
-        }
-        if (wc == q && lb == o) {
+        for (int h = 0; h < 2; ++h) {  // the buffers' parity
+          const int o = o2 + h, i = i0 + o;
+          if (i >= N) break;
+          if (wr == q && la == o) {
 #pragma unroll
-          for (int r = 0; r < T; ++r) colb[r0 + 8 * r] = g[r][k];
-        }
-        __syncthreads();
-        const double gu = pb[i], gd = pb[NP + i], u = ub[i], ep = e2[i];
-        double x[T], y[T];
-#pragma unroll
-        for (int r = 0; r < T; ++r) x[r] = colb[r0 + 8 * r];
-#pragma unroll
-        for (int j = 0; j < T; ++j) y[j] = rowb[c0 + 8 * j];
-        const double em = ep == ch.e2p ? ch.e2m : ch.e2p;
-        const double d_up = 1.0 + (1.0 - gu) * (ep - 1.0);
-        const double d_dn = 1.0 + (1.0 - gd) * (em - 1.0);
-        const double ratio = d_up * d_dn;
-        const bool acc = u <= ratio;
-        if (!isfinite(ratio)) bad = true;
-        if (tid == 0) {
-          acc_sh[i] = acc ? 1 : 0;
-          if (a.trace) red[i] = ratio;
-        }
-        if (acc) {
-          ++nacc;
-          // y = e_i - G[i, :], coefficient alpha / (1 + alpha (1 - G_ii)) of my spin
-          const double cf = sp == 0 ? ft_div(ep - 1.0, d_up) : ft_div(em - 1.0, d_dn);
-          double cy[T];
-#pragma unroll
-          for (int j = 0; j < T; ++j) {
-            const double yj = c0 + 8 * j == i ? 1.0 - y[j] : -y[j];
-            cy[j] = cf * yj;
+            for (int j = 0; j < T; ++j) rowb[h * PB + 8 * j] = g[k][j];
           }
+          if (wc == q && lb == o) {
 #pragma unroll
-          for (int r = 0; r < T; ++r)
+            for (int r = 0; r < T; ++r) colb[h * PB + 8 * r] = g[r][k];
+          }
+          const double u = ft_readlane(ul, o);
+          const bool neg = __builtin_amdgcn_readlane(nl, o) != 0;
+          const double al_up = neg ? am : ap, al_dn = neg ? ap : am;
+          __syncthreads();
+          const double gu = buf[h * PB + i], gd = buf[h * PB + NP + i];
+          double x[T], y[T];
 #pragma unroll
-            for (int j = 0; j < T; ++j) g[r][j] = fma(-cy[j], x[r], g[r][j]);
+          for (int r = 0; r < T; ++r) x[r] = colb[h * PB + 8 * r];
+#pragma unroll
+          for (int j = 0; j < T; ++j) y[j] = rowb[h * PB + 8 * j];
+          const double d_up = 1.0 + (1.0 - gu) * al_up;
+          const double d_dn = 1.0 + (1.0 - gd) * al_dn;
+          const double ratio = d_up * d_dn;
+          if (a.trace && tid == 0) red[i] = ratio;
+          fin = fma(ratio, 0.0, fin);
+          if (u <= ratio) {
+            ++nacc;
+            abits |= 1u << o;
+            // G -= x (cf y)^T, y = e_i - G[i, :], cf = alpha / (1 + alpha (1 - G_ii)) of my spin
+            const double cf = ft_div(sp == 0 ? al_up : al_dn, sp == 0 ? d_up : d_dn);
+            if (wc == q && lb == o) y[k] -= 1.0;
+#pragma unroll
+            for (int j = 0; j < T; ++j) y[j] = cf * y[j];
+#pragma unroll
+            for (int r = 0; r < T; ++r)
+#pragma unroll
+              for (int j = 0; j < T; ++j) g[r][j] = fma(y[j], x[r], g[r][j]);
+          }
         }
       }
+      if (tid == 0) acc_sh[i0 >> 3] = (int)abits;
     }
   }
   {
@@ -149,13 +165,14 @@ __global__ __launch_bounds__(128 * WR * WR) void k_flip_tile(FlipArgs a) {
   }
   __syncthreads();
   for (int i = tid; i < N; i += blockDim.x) {
+    const int acc = (acc_sh[i >> 3] >> (i & 7)) & 1;
     if (a.trace) {
       ch.tr_ratio[(size_t)a.t * N + i] = red[i];
-      ch.tr_acc[(size_t)a.t * N + i] = (uint8_t)acc_sh[i];
+      ch.tr_acc[(size_t)a.t * N + i] = (uint8_t)acc;
     }
-    if (acc_sh[i]) fld[i] = (int8_t)(-fld[i]);
+    if (acc) fld[i] = (int8_t)(neg_sh[i] ? 1 : -1);
   }
-  slice_epilogue<double>(a, ch, c, l, G, nacc, underrun, bad, red);
+  slice_epilogue<double>(a, ch, c, l, G, nacc, underrun, !(fin == 0.0), red);
 }
 
 // Sites covered by class k of the kernel's forms (rising; the last one is the limit of its use).
@@ -171,7 +188,7 @@ int flip_tile_class(int N) {
 template <int T, int WR>
 static void ft_launch(const FlipArgs& a, hipStream_t s) {
   constexpr int threads = 128 * WR * WR, NP = 8 * T * WR;
-  const size_t sh = sizeof(double) * (8 * NP + 2 * NP + std::max(threads, NP)) + NP;
+  const size_t sh = sizeof(double) * (9 * NP + std::max(threads, NP)) + sizeof(int) * (NP + NP / 8);
   hipLaunchKernelGGL((k_flip_tile<T, WR>), dim3(a.nchains), dim3(threads), sh, s, a);
 }
 

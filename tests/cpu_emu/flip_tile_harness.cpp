@@ -54,7 +54,7 @@ static Batch make(int N, int L, int nch, double gscale) {
 template <int T, int WR>
 static void run(FlipArgs a, int nch) {
   constexpr int threads = 128 * WR * WR, NP = 8 * T * WR;
-  const size_t sh = sizeof(double) * (10 * NP + std::max(threads, NP)) + NP;
+  const size_t sh = sizeof(double) * (9 * NP + std::max(threads, NP)) + sizeof(int) * (NP + NP / 8);
   emu_launch(nch, threads, sh, [&] { k_flip_tile<T, WR>(a); });
 }
 
