@@ -876,6 +876,15 @@ int lqmc_create(lqmc_ctx** out, int device, int n_chains, const int32_t* n_sites
       // at least one 16-row strip of either spin per wavefront
       const int strips = 2 * ((nmax_flip + 15) / 16);
       x->flip_groups = std::max(1, std::min(cus / padded, strips / waves));
+      // 16-site blocks with compute units to spare: twice the workgroups of four wavefronts, each
+      // alone on its SIMD (one 16 x 16 chain: 362 us per launch as 4 x 512 threads, 330 as 8 x 256,
+      // 339 as 16 x 256, 374 as 8 x 512; eight chains 370 and 341)
+      const int wide = std::min(cus / padded, strips / 4);
+      if (o.delay == 16 && o.flip_threads <= 0 && waves == 8 && wide >= 2 * x->flip_groups) {
+        x->flip_groups = 2 * x->flip_groups;
+        x->flip_threads = 256;
+        x->flip_shmem = flip_delayed_shmem(nmax_flip, o.delay, x->flip_threads, fp32);
+      }
     } else if (splittable) {
       // rank-1: at least 32 rows of each spin per workgroup
       x->flip_groups = std::max(1, std::min(cus / padded, nmax_flip / 32));
