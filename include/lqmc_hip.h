@@ -80,7 +80,7 @@ typedef struct {
   int32_t dense_ek;    /* 1: every product with E_K or E_K^-1 as a dense GEMM.  0 (default): where
                           E_K = Ex (x) Ey and E_K^-1 = Exi (x) Eyi exactly (a hopping matrix that is
                           a Kronecker sum, e.g. the square and cubic lattices; checked entry by
-                          entry to 1e-13 of max|E_K| in lqmc_set_chain, n1, n2 <= 16), the FP64
+                          entry to 1e-13 of max|E_K| in lqmc_set_chain, n1, n2 <= 32), the FP64
                           products apply the factors: 2 N^2 (n1 + n2) flops in place of 2 N^3,
                           equal to the dense product up to rounding. */
 } lqmc_options;

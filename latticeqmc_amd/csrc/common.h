@@ -7,6 +7,9 @@
 // Global address space: loads through such pointers are global_load (vector-memory
 // counter only) rather than flat loads, which also hold the LDS counter.
 #define LQMC_GLOBAL __attribute__((address_space(1)))
+// Constant address space: memory that no kernel of the launch writes, read through scalar loads
+// where the address is the same in every lane.
+#define LQMC_CONST __attribute__((address_space(4)))
 // The value of x (in an SGPR: "s", a VGPR: "v") passed through an empty asm: expressions
 // formed from it afterwards are new to the compiler and are not merged with earlier ones.
 #define LQMC_OPAQUE(x, reg) asm volatile("" : "+" reg(x))
@@ -14,6 +17,7 @@
 #define LQMC_WAVE_PRIO(p) __builtin_amdgcn_s_setprio(p)
 #else
 #define LQMC_WAVE_PRIO(p) ((void)0)
+#define LQMC_CONST
 #endif
 #include <stdint.h>
 
@@ -123,8 +127,9 @@ struct GemmTask {
 };
 
 // C = diag(rs) E diag(ks) X diag(cs) (left) or C = diag(rs) X diag(ks) E diag(cs) (right) for
-// a Kronecker-factored E = Ex (x) Ey (site i = a n2 + b; Ex n1 x n1, Ey n2 x n2, n1, n2 <= 16,
-// each stored as a 16 x 16 row-major block, zero outside).  X and C are N x N, N = n1 n2.
+// a Kronecker-factored E = Ex (x) Ey (site i = a n2 + b; Ex n1 x n1, Ey n2 x n2), N = n1 n2, X and
+// C N x N.  k_kron: n1, n2 <= 16, the factors 16 x 16 row-major blocks, zero outside.  k_kron_wide:
+// n1, n2 <= 32, the factors 32 x 32 blocks, transposed for the right product.
 struct KronTask {
   const double* X;
   double* C;

@@ -30,6 +30,10 @@ namespace lqmc {
 void launch_gemm(int fp32, int cls, const GemmTask* d_tasks, int ntasks, int ntiles, hipStream_t s);
 void launch_kron(int right, int all16, const KronTask* d_tasks, int ntasks, int ntiles, int cus, hipStream_t s);
 int kron_tiles(int N);
+void launch_kron_wide(int right, const KronTask* d_tasks, int ntasks, int ntiles, int threads, size_t shmem,
+                      hipStream_t s);
+int kron_wide_threads(int n1, int n2);
+size_t kron_wide_shmem(int n1, int n2);
 int gemm_class(const GemmTask& t);
 int gemm_tiles(int M, int N, int* tiles_n);
 void launch_qr_blocked(const QrTask* d, int n, int nmax, ChainState* st, unsigned* pub, int max_wg, hipStream_t s);
@@ -80,7 +84,7 @@ static int fail(int code, const std::string& msg) {
 
 namespace {
 
-enum OpKind { OP_GEMM = 0, OP_QR, OP_SOLVE, OP_FINISH, OP_FLIP, OP_EXPV, OP_IDENT, OP_TRSM, OP_DET, OP_KRON };
+enum OpKind { OP_GEMM = 0, OP_QR, OP_SOLVE, OP_FINISH, OP_FLIP, OP_EXPV, OP_IDENT, OP_TRSM, OP_DET, OP_KRON, OP_KRON_WIDE };
 enum ProfKind { PK_FLIP = 0, PK_GEMM = 1, PK_QR = 2, PK_SOLVE = 3, PK_KRON = 4 };
 
 struct Op {
@@ -93,6 +97,8 @@ struct Op {
   int t;
   double work;  // algorithmic work units (flips for OP_FLIP, flops for OP_GEMM)
   int meas_only = 0;  // skipped in sweeps that do not measure
+  int threads = 0;    // OP_KRON_WIDE: launch shape
+  size_t shmem = 0;
 };
 
 struct Chain {
@@ -109,9 +115,10 @@ struct Chain {
   uint8_t* tr_acc = nullptr;
   double *expk = nullptr, *expki = nullptr;
   float *expk32 = nullptr, *expki32 = nullptr;
-  // E_K = Ex (x) Ey and E_K^-1 = Exi (x) Eyi when the lattice factors (kn1 > 0): the four
-  // 16 x 16 blocks Ex, Ey, Exi, Eyi at kr, zero-padded
-  int kn1 = 0, kn2 = 0;
+  // E_K = Ex (x) Ey and E_K^-1 = Exi (x) Eyi when the lattice factors (kn1 > 0): the eight blocks
+  // Ex, Ey, Exi, Eyi and their transposes at kr, kdim x kdim (16, or 32 with a longer direction),
+  // zero-padded
+  int kn1 = 0, kn2 = 0, kdim = 16;
   double* kr = nullptr;
   double *Wa[2] = {}, *Wb[2] = {};
   double *LU[2] = {}, *LD[2] = {}, *LV[2] = {};
@@ -171,6 +178,7 @@ struct lqmc_ctx {
   unsigned* d_bar = nullptr;     // [nchains][4] their barrier counters and XCC bits
   unsigned* d_qrpub = nullptr;   // [4 nchains] hand-over counters of the on-chip QR (two per matrix)
   int cus = 0;                   // compute units of the device
+  size_t lds = 0;                // its LDS per workgroup
   size_t flip_shmem = 0;
   size_t det_shmem = 0;
   // graphs
@@ -218,7 +226,7 @@ static void layout_chain(const lqmc_ctx* x, Chain& c, char* base, size_t& off) {
     carve(base, off, c.expk32, n2);
     carve(base, off, c.expki32, n2);
   }
-  carve(base, off, c.kr, 4 * 256);
+  carve(base, off, c.kr, 8 * (N >= 34 ? 1024 : 256));  // 34 = 2 * 17 sites: the smallest wide lattice
   carve(base, off, c.eye, n2);
   carve(base, off, c.ones, N);
   if (x->opt.delay > 1) {
@@ -289,8 +297,9 @@ struct Builder {
       k = KronTask{};
       k.X = static_cast<const double*>(la ? t.B : t.A);
       k.C = static_cast<double*>(t.C);
-      k.Ex = c.kr + (inv ? 512 : 0);
-      k.Ey = c.kr + (inv ? 768 : 256);
+      const int blk = c.kdim * c.kdim, first = (inv ? 2 : 0) + (right && c.kdim == 32 ? 4 : 0);
+      k.Ex = c.kr + first * blk;
+      k.Ey = c.kr + (first + 1) * blk;
       k.rs = t.rs; k.ks = t.ks; k.cs = t.cs;
       k.rs_kind = t.rs_kind; k.ks_kind = t.ks_kind; k.cs_kind = t.cs_kind;
       k.N = c.N; k.n1 = c.kn1; k.n2 = c.kn2;
@@ -304,13 +313,26 @@ struct Builder {
   void gemm(std::vector<Op>& ops, std::vector<GemmTask>& tasks, int fp32) {
     if (tasks.empty()) return;
     {
-      std::vector<KronTask> kt[2];
+      std::vector<KronTask> kt[2], wide[2];
       std::vector<GemmTask> rest;
       for (auto& t : tasks) {
         KronTask k;
         int right = 0;
-        if (as_kron(t, fp32, k, right)) kt[right].push_back(k);
+        if (as_kron(t, fp32, k, right)) (std::max(k.n1, k.n2) > 16 ? wide : kt)[right].push_back(k);
         else rest.push_back(t);
+      }
+      for (int right = 0; right < 2; ++right) {
+        if (wide[right].empty()) continue;
+        Op op{OP_KRON_WIDE, 0, 0, (int)wide[right].size(), 0, right, 0, 0.0};
+        for (auto& k : wide[right]) {
+          k.tile_base = op.ntiles;
+          op.ntiles += kron_tiles(k.N);
+          op.work += 2.0 * k.N * (double)k.N * (k.n1 + k.n2);
+          op.threads = std::max(op.threads, kron_wide_threads(k.n1, k.n2));
+          op.shmem = std::max(op.shmem, kron_wide_shmem(k.n1, k.n2));
+        }
+        op.off = push(wide[right]);
+        ops.push_back(op);
       }
       for (int right = 0; right < 2; ++right) {
         if (kt[right].empty()) continue;
@@ -702,7 +724,7 @@ static void run_ops(lqmc_ctx* x, const std::vector<Op>& ops, int measure, hipStr
     else if (op.kind == OP_GEMM) pk = PK_GEMM;
     else if (op.kind == OP_QR) pk = PK_QR;
     else if (op.kind == OP_SOLVE || op.kind == OP_TRSM) pk = PK_SOLVE;
-    else if (op.kind == OP_KRON) pk = PK_KRON;
+    else if (op.kind == OP_KRON || op.kind == OP_KRON_WIDE) pk = PK_KRON;
     const bool rec = profile && pk == x->prof.kind;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (rec) {
@@ -714,6 +736,9 @@ static void run_ops(lqmc_ctx* x, const std::vector<Op>& ops, int measure, hipStr
     switch (op.kind) {
       case OP_GEMM: launch_gemm(op.fp32, op.nmax, reinterpret_cast<const GemmTask*>(d), op.count, op.ntiles, s); break;
       case OP_KRON: launch_kron(op.nmax, op.fp32, reinterpret_cast<const KronTask*>(d), op.count, op.ntiles, x->cus, s); break;
+      case OP_KRON_WIDE:
+        launch_kron_wide(op.nmax, reinterpret_cast<const KronTask*>(d), op.count, op.ntiles, op.threads, op.shmem, s);
+        break;
       case OP_QR:
         launch_qr_blocked(reinterpret_cast<const QrTask*>(d), op.count, op.nmax, x->d_state, x->d_qrpub, x->cus, s);
         break;
@@ -851,7 +876,7 @@ int lqmc_create(lqmc_ctx** out, int device, int n_chains, const int32_t* n_sites
     }
     const int cus = prop.multiProcessorCount;
     x->cus = cus;
-    lds_dev = prop.sharedMemPerBlock;
+    lds_dev = x->lds = prop.sharedMemPerBlock;
     const int nflip = nrest ? nrest : n_chains;
     const int padded = 8 * ((nflip + 7) / 8);
     const bool splittable = o.mode == LQMC_MODE_DQMC && (o.delay == 1 || o.delay == 16 || o.delay == 32);
@@ -999,23 +1024,24 @@ static void refresh_chain_desc(lqmc_ctx* x, int ci) {
 // off the first rows of blocks, Ex[a][a'] = E[a n2][a' n2] and Ey[b][b'] = E[b][b'] / E[0][0] (so
 // that Ex[a][a'] Ey[b][b'] = E[a n2][a' n2] E[b][b'] / E[0][0]), and accepted when every entry of
 // E matches its Kronecker product to 1e-13 of max|E|: an E_K = expm(-dtau K) of a hopping matrix
-// K = Kx (x) I + I (x) Ky does (the two terms commute), any other fails.  f: [Ex | Ey] as 16 x 16
+// K = Kx (x) I + I (x) Ky does (the two terms commute), any other fails.  f: [Ex | Ey] as dim x dim
 // row-major blocks, zero outside.
-static bool kron_factor(const double* E, int N, int n2, double* f) {
+static bool kron_factor(const double* E, int N, int n2, int dim, double* f) {
   const int n1 = N / n2;
   const double e00 = E[0];
   if (!(e00 > 0.0)) return false;
   double emax = 0.0;
   for (size_t e = 0; e < (size_t)N * N; ++e) emax = std::max(emax, std::fabs(E[e]));
-  std::fill(f, f + 512, 0.0);
+  double* fy = f + dim * dim;
+  std::fill(f, fy + dim * dim, 0.0);
   for (int a = 0; a < n1; ++a)
-    for (int a2 = 0; a2 < n1; ++a2) f[a * 16 + a2] = E[(size_t)a * n2 * N + (size_t)a2 * n2];
+    for (int a2 = 0; a2 < n1; ++a2) f[a * dim + a2] = E[(size_t)a * n2 * N + (size_t)a2 * n2];
   for (int b = 0; b < n2; ++b)
-    for (int b2 = 0; b2 < n2; ++b2) f[256 + b * 16 + b2] = E[(size_t)b * N + b2] / e00;
+    for (int b2 = 0; b2 < n2; ++b2) fy[b * dim + b2] = E[(size_t)b * N + b2] / e00;
   const double tol = 1e-13 * emax;
   for (int i = 0; i < N; ++i)
     for (int k = 0; k < N; ++k) {
-      const double p = f[(i / n2) * 16 + k / n2] * f[256 + (i % n2) * 16 + k % n2];
+      const double p = f[(i / n2) * dim + k / n2] * fy[(i % n2) * dim + k % n2];
       if (!(std::fabs(E[(size_t)i * N + k] - p) <= tol)) return false;
     }
   return true;
@@ -1047,22 +1073,29 @@ int lqmc_set_chain(lqmc_ctx* x, int ci, const double* expk, const double* expk_i
   HIPCHK(hipMemcpy(c.hop, hop.data(), n2 * 8, hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(c.eye, eye.data(), n2 * 8, hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(c.ones, ones.data(), N * 8, hipMemcpyHostToDevice));
-  // Kronecker factors of E_K and E_K^-1 (the first split N = n1 n2, 2 <= n1, n2 <= 16, largest
-  // n2 first, that both admit), unless dense products are asked for
+  // Kronecker factors of E_K and E_K^-1 (the first split N = n1 n2 that both admit, largest n2 first,
+  // 2 <= n1, n2 <= 16, then those with a direction of up to 32 where its tiles fit the device's LDS),
+  // unless dense products are asked for
   c.kn1 = c.kn2 = 0;
   if (!x->opt.dense_ek && x->opt.mode != LQMC_MODE_DET) {
-    std::vector<double> kf(1024);
-    for (int n2c = 16; n2c >= 2; --n2c) {
-      if ((int)N % n2c != 0) continue;
-      const int n1c = (int)N / n2c;
-      if (n1c < 2 || n1c > 16) continue;
-      if (kron_factor(expk, (int)N, n2c, kf.data()) && kron_factor(expk_inv, (int)N, n2c, kf.data() + 512)) {
-        c.kn1 = n1c;
-        c.kn2 = n2c;
-        break;
+    std::vector<double> kf(8 * 1024);
+    for (int dim = 16; dim <= 32 && !c.kn1; dim += 16)
+      for (int n2c = dim; n2c >= 2; --n2c) {
+        if ((int)N % n2c != 0) continue;
+        const int n1c = (int)N / n2c, blk = dim * dim;
+        if (n1c < 2 || n1c > dim || (dim == 32 && std::max(n1c, n2c) <= 16)) continue;
+        if (dim == 32 && kron_wide_shmem(n1c, n2c) > x->lds) continue;
+        if (kron_factor(expk, (int)N, n2c, dim, kf.data()) && kron_factor(expk_inv, (int)N, n2c, dim, kf.data() + 2 * blk)) {
+          for (int m = 0; m < 4; ++m)
+            for (int r = 0; r < dim; ++r)
+              for (int q = 0; q < dim; ++q) kf[(4 + m) * blk + q * dim + r] = kf[m * blk + r * dim + q];
+          c.kn1 = n1c;
+          c.kn2 = n2c;
+          c.kdim = dim;
+          break;
+        }
       }
-    }
-    if (c.kn1) HIPCHK(hipMemcpy(c.kr, kf.data(), 1024 * 8, hipMemcpyHostToDevice));
+    if (c.kn1) HIPCHK(hipMemcpy(c.kr, kf.data(), 8 * (size_t)c.kdim * c.kdim * 8, hipMemcpyHostToDevice));
   }
   if (x->opt.precision != LQMC_FP64) {
     std::vector<float> a(n2), b(n2);

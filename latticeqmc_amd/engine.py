@@ -72,7 +72,7 @@ class SweepEngine:
     max_dg    Mode D: a recompute deviating from the propagated G by more than this raises
               a device flag, so ``sync`` fails (0: 1e-3; negative: off)
     dense_ek  run every product with E_K as a dense GEMM; by default a chain whose E_K is
-              exactly Ex (x) Ey (square and cubic lattices, n1, n2 <= 16) applies the factors
+              exactly Ex (x) Ey (square and cubic lattices, n1, n2 <= 32) applies the factors
               in its FP64 products (``ek_split``)
     """
 
