@@ -38,7 +38,7 @@ def flags():
 # Per-source extra flags.  gemm.hip: keep the matrix-core accumulators in VGPRs (the default
 # AGPR form copied all 32 accumulator registers between the two files on every k-tile of the
 # GEMM loop).
-EXTRA = {"gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+EXTRA = {"gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"], "flip_tile.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 
 PROBE_LIB = os.path.join(HERE, "liblqmc_hip_probe.so")

@@ -26,6 +26,18 @@ __device__ inline LQMC_GLOBAL T* gptr(T* p) {
   return (LQMC_GLOBAL T*)p;
 }
 
+// A pointer that is the same in every lane, in scalar registers.
+template <typename T>
+__device__ inline const LQMC_CONST T* uniform_const(const T* p) {
+#ifdef LQMC_CPU_EMU
+  return p;
+#else
+  const uint64_t b = (uint64_t)p;
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)b), hi = __builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));
+  return (const LQMC_CONST T*)(((uint64_t)hi << 32) | lo);
+#endif
+}
+
 // Block index regrouped by XCD.  Workgroups are dispatched to the eight XCDs round-robin
 // (block b on XCD b % 8), each XCD with its own L2.  The returned index runs consecutively
 // over the blocks of one XCD, so neighbouring indices (the tiles or column blocks of one
@@ -75,7 +87,8 @@ struct ChainDev {
   double* obs;         // [obs_cap][3]
   void* dws;           // delayed-update workspace: Z tiles of both spins in register order
   int obs_cap;
-  int pad1;
+  int kn1, kn2;        // sites of the two lattice directions of the factored E_K (flips with wraps)
+  const double* kr;    // its 16 x 16 blocks Ex, Ey, Exi, Eyi, then their transposes
 };
 
 // Mutable per-chain counters (device).
@@ -209,6 +222,7 @@ struct FlipArgs {
   int yrows;      // delayed flip, k = 16, one spin per workgroup: the block's rows of G and its Z tiles
                   // kept in LDS (flip_delayed_stage_rows; flip_delayed_rows_shmem more bytes of LDS)
   const int* list;  // the launch's nchains chains (null: chains 0 .. nchains-1)
+  int slices;       // register-tile flip with wraps: slices t .. t + slices - 1 in one launch
 };
 
 }  // namespace lqmc

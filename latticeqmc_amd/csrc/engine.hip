@@ -48,6 +48,7 @@ void launch_flip(int fp32, int delayed, const FlipArgs& a, int nchains, int thre
                  hipStream_t s);
 void launch_flip_tile(int cls, const FlipArgs& a, hipStream_t s);
 int flip_tile_class(int N);
+size_t flip_tile_wrap_shmem(int cls);
 size_t flip_delayed_shmem(int nmax, int k, int threads, int fp32);
 size_t flip_delayed_workspace(int n, int k, int fp32, int groups);
 int flip_delayed_stage_rows(int nmax, int k, int groups);
@@ -119,6 +120,7 @@ struct Chain {
   // Ex, Ey, Exi, Eyi and their transposes at kr, kdim x kdim (16, or 32 with a longer direction),
   // zero-padded
   int kn1 = 0, kn2 = 0, kdim = 16;
+  bool fused = false;  // flips and wraps of a stabilisation block in one launch
   double* kr = nullptr;
   double *Wa[2] = {}, *Wb[2] = {};
   double *LU[2] = {}, *LD[2] = {}, *LV[2] = {};
@@ -167,11 +169,14 @@ struct lqmc_ctx {
   double** d_eye_ptrs = nullptr;
   int* d_eye_ns = nullptr;
   int nmax = 0, lmax = 0;
-  // flips: chains [tile_off[k], tile_off[k+1]) of the list in the register-tile form of class k, the
-  // others (from tile_off[8] on) in the form that the options name
+  // flips: chains [tile_off[w][k], tile_off[w][k+1]) of the list in the register-tile form of class k,
+  // w = 1 with their wraps (fused), w = 0 without; the others (from tile_off[0][8] on) in the form that
+  // the options name
   int* d_flip_list = nullptr;
-  int tile_off[9] = {};
-  int flip_rest = 0;             // chains from tile_off[8] on
+  std::vector<int> flip_list;
+  int tile_off[2][9] = {};
+  int flip_rest = 0;             // chains from tile_off[0][8] on
+  bool tiled = false;            // the options leave chains of up to 128 sites to the register-tile form
   int flip_threads = 256;
   int flip_groups = 1;           // workgroups per chain of the delayed flip
   int flip_yrows = 0;            // delayed flip keeps block rows and Z tiles in LDS (FlipArgs::yrows)
@@ -414,7 +419,36 @@ GemmTask mk(const void* A, int lda, int tA, const void* B, int ldb, int tB, void
 
 }  // namespace
 
+// Flip launches: chains up to 128 sites in the register-tile form, with the wraps where E_K factors into
+// directions of up to 16 sites.  One launch per class present, or a single one in the largest class while
+// every chain has a compute unit to itself (the launch then takes as long as its slowest chain either way).
+static void flip_lists(lqmc_ctx* x) {
+  std::vector<int>& list = x->flip_list;
+  list.clear();
+  std::vector<int> cls(x->nchains, -1);
+  for (int c = 0; c < x->nchains; ++c) {
+    Chain& h = x->ch[c];
+    if (x->tiled) cls[c] = flip_tile_class(h.N);
+    h.fused = cls[c] >= 0 && h.kn1 > 0 && h.kdim == 16 && flip_tile_wrap_shmem(7) <= x->lds;
+  }
+  for (int w = 1; w >= 0; --w) {
+    int top = -1, count = 0;
+    for (int c = 0; c < x->nchains; ++c)
+      if (cls[c] >= 0 && x->ch[c].fused == (w == 1)) { ++count; top = std::max(top, cls[c]); }
+    for (int k = 0; k < 8; ++k) {
+      x->tile_off[w][k] = (int)list.size();
+      for (int c = 0; c < x->nchains; ++c)
+        if (cls[c] >= 0 && x->ch[c].fused == (w == 1) && (count <= x->cus ? top : cls[c]) == k) list.push_back(c);
+    }
+    x->tile_off[w][8] = (int)list.size();
+  }
+  x->flip_rest = 0;
+  for (int c = 0; c < x->nchains; ++c)
+    if (cls[c] < 0) { list.push_back(c); ++x->flip_rest; }
+}
+
 static void build_program(lqmc_ctx* x) {
+  flip_lists(x);
   x->h_desc.clear();
   x->init_ops.clear();
   x->sweep_ops.clear();
@@ -434,9 +468,14 @@ static void build_program(lqmc_ctx* x) {
   x->init_ops.push_back(Op{OP_IDENT, 0, 0, nc, 0, 0, 0, 0});
 
   auto flipop = [&](std::vector<Op>& ops, int t) {
+    if (t % ns == 0) {  // the block's flips and wraps of the fused chains
+      double w = 0;
+      for (auto& c : x->ch) if (c.fused) w += c.N * (double)std::max(0, std::min(ns, c.L - t));
+      if (w > 0) ops.push_back(Op{OP_FLIP, fp32, 0, nc, 0, ns, t, w});
+    }
     double w = 0;
-    for (auto& c : x->ch) if (t < c.L) w += c.N;
-    ops.push_back(Op{OP_FLIP, fp32, 0, nc, 0, 0, t, w});
+    for (auto& c : x->ch) if (!c.fused && t < c.L) w += c.N;
+    if (w > 0) ops.push_back(Op{OP_FLIP, fp32, 0, nc, 0, 0, t, w});
   };
   auto evp = [&](Chain& c, int s, int l) { return c.ev + (size_t)s * c.N * c.L + (size_t)l * c.N; };
   auto evip = [&](Chain& c, int s, int l) { return c.evi + (size_t)s * c.N * c.L + (size_t)l * c.N; };
@@ -654,7 +693,7 @@ static void build_program(lqmc_ctx* x) {
       flipop(x->sweep_ops, t);
       for (int ci = 0; ci < nc; ++ci) {
         Chain& c = x->ch[ci];
-        if (t >= c.L) continue;
+        if (t >= c.L || c.fused) continue;
         const int l = c.L - 1 - t;
         for (int s = 0; s < 2; ++s) {
           const void* ekinv = fp32 ? (const void*)c.expki32 : (const void*)c.expki;
@@ -753,15 +792,17 @@ static void run_ops(lqmc_ctx* x, const std::vector<Op>& ops, int measure, hipStr
       case OP_FLIP: {
         FlipArgs a{x->d_chains, x->d_state, op.t, measure, x->opt.rng, x->opt.trace, x->opt.delay,
                    x->flip_groups, x->d_bar, x->nchains, x->opt.precision == LQMC_BF16X3 ? 1 : 0,
-                   x->flip_yrows, nullptr};
+                   x->flip_yrows, nullptr, 0};
+        const int* off = x->tile_off[op.nmax > 0 ? 1 : 0];  // op.nmax: slices of the fused chains' launch
+        a.slices = op.nmax;
         for (int k = 0; k < 8; ++k) {
-          a.nchains = x->tile_off[k + 1] - x->tile_off[k];
-          a.list = x->d_flip_list + x->tile_off[k];
+          a.nchains = off[k + 1] - off[k];
+          a.list = x->d_flip_list + off[k];
           launch_flip_tile(k, a, s);
         }
-        if (x->flip_rest) {
+        if (op.nmax == 0 && x->flip_rest) {
           a.nchains = x->flip_rest;
-          a.list = x->d_flip_list + x->tile_off[8];
+          a.list = x->d_flip_list + off[8];
           launch_flip(fp32, x->opt.delay > 1, a, x->flip_rest, x->flip_threads, x->flip_shmem, s);
         }
         break;
@@ -834,6 +875,7 @@ int lqmc_create(lqmc_ctx** out, int device, int n_chains, const int32_t* n_sites
   // FP64 Mode D chains of up to 128 sites flip in registers (flip_tile.hip) unless the options name a
   // form of the other flip kernels; nrest / nmax_rest: the chains left to those.
   const bool tiled = o.mode == LQMC_MODE_DQMC && o.precision == LQMC_FP64 && o.flip_threads == 0 && o.flip_groups == 0;
+  x->tiled = tiled;
   int nrest = 0, nmax_rest = 0;
   for (auto& c : x->ch)
     if (!tiled || flip_tile_class(c.N) < 0) { ++nrest; nmax_rest = std::max(nmax_rest, c.N); }
@@ -969,28 +1011,9 @@ int lqmc_create(lqmc_ctx** out, int device, int n_chains, const int32_t* n_sites
   off = 0;
   for (auto& c : x->ch) layout_chain(x, c, x->arena, off);
   x->h_chains.resize(n_chains);
-  {
-    // Flip launches: one per class present, or a single one in the largest class while every chain has
-    // a compute unit to itself (the launch then takes as long as its slowest chain either way).
-    std::vector<int> list, cls(n_chains, -1);
-    int top = -1;
-    for (int c = 0; c < n_chains; ++c)
-      if (tiled) { cls[c] = flip_tile_class(x->ch[c].N); top = std::max(top, cls[c]); }
-    const bool one = n_chains - nrest <= x->cus;
-    for (int k = 0; k < 8; ++k) {
-      x->tile_off[k] = (int)list.size();
-      for (int c = 0; c < n_chains; ++c)
-        if (cls[c] >= 0 && (one ? top : cls[c]) == k) list.push_back(c);
-    }
-    x->tile_off[8] = (int)list.size();
-    x->flip_rest = nrest;
-    for (int c = 0; c < n_chains; ++c)
-      if (cls[c] < 0) list.push_back(c);
-    if (hipMalloc(&x->d_flip_list, sizeof(int) * n_chains) != hipSuccess ||
-        hipMemcpy(x->d_flip_list, list.data(), sizeof(int) * n_chains, hipMemcpyHostToDevice) != hipSuccess) {
-      lqmc_destroy(x);
-      return fail(LQMC_ENOMEM, "flip list allocation failed");
-    }
+  if (hipMalloc(&x->d_flip_list, sizeof(int) * n_chains) != hipSuccess) {
+    lqmc_destroy(x);
+    return fail(LQMC_ENOMEM, "flip list allocation failed");
   }
   std::vector<double*> eyes(n_chains);
   std::vector<int> ns(n_chains);
@@ -1017,6 +1040,7 @@ static void refresh_chain_desc(lqmc_ctx* x, int ci) {
   d.expk = c.expk;
   d.tr_ratio = c.tr_ratio; d.tr_acc = c.tr_acc; d.obs = c.obs; d.obs_cap = x->opt.obs_capacity;
   d.dws = c.dws;
+  d.kn1 = c.kn1; d.kn2 = c.kn2; d.kr = c.kr;
   x->h_chains[ci] = d;
 }
 
@@ -1178,6 +1202,7 @@ int lqmc_init(lqmc_ctx* x) {
   build_program(x);
   int rc = upload_program(x);
   if (rc) return rc;
+  HIPCHK(hipMemcpy(x->d_flip_list, x->flip_list.data(), sizeof(int) * x->nchains, hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(x->d_chains, x->h_chains.data(), sizeof(ChainDev) * x->nchains, hipMemcpyHostToDevice));
   run_ops(x, x->init_ops, 0, x->stream, false);
   HIPCHK(hipGetLastError());

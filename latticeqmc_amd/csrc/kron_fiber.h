@@ -8,18 +8,6 @@
 
 namespace lqmc {
 
-// A pointer that is the same in every lane, in scalar registers.
-template <typename T>
-__device__ inline const LQMC_CONST T* uniform_const(const T* p) {
-#ifdef LQMC_CPU_EMU
-  return p;
-#else
-  const uint64_t b = (uint64_t)p;
-  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)b), hi = __builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));
-  return (const LQMC_CONST T*)(((uint64_t)hi << 32) | lo);
-#endif
-}
-
 // v[b st] <- sum_k E[b ld + k] v[k st], b, k < n; n is F or F - 1 (E is zero past n up to row and column F).
 template <int F>
 __device__ __attribute__((always_inline)) inline void kf_fiber(double* v, int st, const LQMC_CONST double* E, int ld, int n) {
