@@ -157,6 +157,21 @@ struct KronTask {
   int tile_base;  // first 16-column (left) or 16-row (right) tile of this task in the launch
 };
 
+// C = S_n .. S_2 S_1 X diag(cs), S_i = diag(rs_i) E diag(ks_i), E as in KronTask (n1, n2 <= 16): the products of
+// a stabilisation block.  The scales are plain; step i reads them i * stride further on (null: none).
+struct KronChainTask {
+  const double* X;
+  double* C;
+  const double* Ex;
+  const double* Ey;
+  const double* rs;
+  const double* ks;
+  const double* cs;
+  int N, n1, n2;
+  int steps, stride;
+  int tile_base;
+};
+
 // Pre-pivoted blocked Householder QR: W = Q diag(D) V'' with V'' written over W.
 struct QrTask {
   double* W;   // in: matrix; out: V'' = D^-1 R P^T, or R' = D^-1 R when perm is requested

@@ -3,12 +3,12 @@
 //
 // A sweep is a fixed sequence of batched launches (all chains, both spins):
 //   Mode D ("dqmc", lqmc/lqmc.py:301-347 made consistent and stabilised)
-//     left stack:  for each slice j bottom-up, W = diag(v_j) E_K W; at the end of
-//                  every block of n_s slices a pivoted QR gives S_m = U D V
+//     left stack:  per block of n_s slices bottom-up, W = diag(v_j) E_K W for its slices, then
+//                  a pivoted QR gives S_m = U D V
 //     for t = 0..L-1 (slice l = L-1-t):
 //        flip(l)                          one workgroup per chain
 //        wrap  G <- E_K^-1 V^-1 G V E_K    two GEMMs (form precision)
-//        right product W <- E_K V W       one FP64 GEMM
+//        right products W <- E_K V W          all of a block at its end
 //        every n_s slices: QR(W), V_R update, stable solve for G(l-1),
 //        compare with the wrapped G and replace it
 //   Mode R ("reference", literal lqmc/lqmc.py:301-347)
@@ -30,6 +30,7 @@ namespace lqmc {
 void launch_gemm(int fp32, int cls, const GemmTask* d_tasks, int ntasks, int ntiles, hipStream_t s);
 void launch_kron(int right, int all16, const KronTask* d_tasks, int ntasks, int ntiles, int cus, hipStream_t s);
 int kron_tiles(int N);
+void launch_kron_chain(int all16, const KronChainTask* d_tasks, int ntasks, int ntiles, hipStream_t s);
 void launch_kron_wide(int right, const KronTask* d_tasks, int ntasks, int ntiles, int threads, size_t shmem,
                       hipStream_t s);
 int kron_wide_threads(int n1, int n2);
@@ -85,7 +86,7 @@ static int fail(int code, const std::string& msg) {
 
 namespace {
 
-enum OpKind { OP_GEMM = 0, OP_QR, OP_SOLVE, OP_FINISH, OP_FLIP, OP_EXPV, OP_IDENT, OP_TRSM, OP_DET, OP_KRON, OP_KRON_WIDE };
+enum OpKind { OP_GEMM = 0, OP_QR, OP_SOLVE, OP_FINISH, OP_FLIP, OP_EXPV, OP_IDENT, OP_TRSM, OP_DET, OP_KRON, OP_KRON_WIDE, OP_KRON_CHAIN };
 enum ProfKind { PK_FLIP = 0, PK_GEMM = 1, PK_QR = 2, PK_SOLVE = 3, PK_KRON = 4 };
 
 struct Op {
@@ -374,6 +375,26 @@ struct Builder {
     }
     tasks.clear();
   }
+  // The left products of a block: diag(rs_i) E_K diag(ks_i) from slice l0 on, steps slices, dl apart.
+  static bool chains(const Chain& c) { return c.kn1 > 0 && c.kdim == 16; }
+  void chain(std::vector<KronChainTask>& tasks, const Chain& c, const double* X, double* C, const double* rs, const double* ks,
+             const double* cs, int dl, int steps) {
+    tasks.push_back(KronChainTask{X, C, c.kr, c.kr + 256, rs, ks, cs, c.N, c.kn1, c.kn2, steps, dl * c.N, 0});
+  }
+  void chain(std::vector<Op>& ops, std::vector<KronChainTask>& tasks) {
+    if (tasks.empty()) return;
+    // fp32 field: whether every task is 16 x 16, as for OP_KRON
+    Op op{OP_KRON_CHAIN, 1, 0, (int)tasks.size(), 0, 0, 0, 0.0};
+    for (auto& k : tasks) {
+      k.tile_base = op.ntiles;
+      op.ntiles += kron_tiles(k.N);
+      op.work += 2.0 * k.steps * k.N * (double)k.N * (k.n1 + k.n2);
+      op.fp32 &= k.n1 == 16 && k.n2 == 16;
+    }
+    op.off = push(tasks);
+    ops.push_back(op);
+    tasks.clear();
+  }
   void qr(std::vector<Op>& ops, std::vector<QrTask>& tasks) {
     if (tasks.empty()) return;
     int nm = 0;
@@ -462,6 +483,7 @@ static void build_program(lqmc_ctx* x) {
   std::vector<SolveTask> sv;
   std::vector<TrsmTask> ts;
   std::vector<FinishTask> fin;
+  std::vector<KronChainTask> kc;
 
   // ---- init: scale tables and identity matrices ----
   x->init_ops.push_back(Op{OP_EXPV, 0, 0, nc, 0, 0, 0, 0});
@@ -542,36 +564,45 @@ static void build_program(lqmc_ctx* x) {
     }
   } else {
     // ---- Mode D ----
-    // left stack: blocks m = nb-1 .. m_min, slices lo..hi (hi = L-1-m*ns)
+    // left stack: blocks m = nb-1 .. m_min, slices lo..hi (hi = L-1-m*ns), every chain's block from the
+    // bottom in the same launches, whatever its number of slices
     auto left_stack = [&](std::vector<Op>& ops, int m_min) {
-      // per chain-spin: which buffer holds the running product
-      std::vector<double*> wcur(nc * 2, nullptr);
-      for (int j = 0; j < x->lmax; ++j) {
-        std::vector<int> ends;
+      int nbmax = 0;
+      for (auto& c : x->ch) nbmax = std::max(nbmax, c.nb);
+      for (int up = 0; up < nbmax; ++up) {
+        std::vector<double*> wcur(nc * 2, nullptr);  // per chain-spin: the buffer that holds the running product
+        for (int k = 0; k < ns; ++k) {
+          for (int ci = 0; ci < nc; ++ci) {
+            Chain& c = x->ch[ci];
+            const int m = c.nb - 1 - up;
+            if (m < m_min) continue;
+            const int lo = std::max(c.L - (m + 1) * ns, 0), hi = c.L - 1 - m * ns, j = lo + k;
+            if (j > hi) continue;
+            const bool bottom = (m == c.nb - 1);
+            for (int s = 0; s < 2; ++s) {
+              double*& w = wcur[ci * 2 + s];
+              const double* first = bottom ? c.eye : c.LU[s] + (size_t)(m + 1) * c.N * c.N;
+              const double* cs = bottom ? nullptr : c.LD[s] + (size_t)(m + 1) * c.N;
+              if (Builder::chains(c)) {
+                if (k == 0) b.chain(kc, c, first, c.Wa[s], evp(c, s, lo), nullptr, cs, 1, hi - lo + 1);
+                w = c.Wa[s];
+                continue;
+              }
+              double* out = (k == 0 || w == c.Wb[s]) ? c.Wa[s] : c.Wb[s];
+              GemmTask g = mk(c.expk, c.N, 0, k == 0 ? first : w, c.N, 0, out, c.N, c.N);
+              g.rs = evp(c, s, j); g.rs_kind = SC_PLAIN;
+              if (k == 0 && cs) { g.cs = cs; g.cs_kind = SC_PLAIN; }
+              g1.push_back(g);
+              w = out;
+            }
+          }
+          b.chain(ops, kc);
+          b.gemm(ops, g1, 0);
+        }
         for (int ci = 0; ci < nc; ++ci) {
           Chain& c = x->ch[ci];
-          const int top = c.L - 1 - m_min * ns;  // last slice in the stack
-          if (j > top) continue;
-          const int m = (c.L - 1 - j) / ns;       // block containing slice j
-          const int lo = std::max(c.L - (m + 1) * ns, 0);
-          const int hi = c.L - 1 - m * ns;
-          for (int s = 0; s < 2; ++s) {
-            double*& w = wcur[ci * 2 + s];
-            double* out = (j == lo || w == c.Wb[s]) ? c.Wa[s] : c.Wb[s];
-            const bool bottom = (m == c.nb - 1);
-            const double* in = (j == lo) ? (bottom ? c.eye : c.LU[s] + (size_t)(m + 1) * c.N * c.N) : w;
-            GemmTask g = mk(c.expk, c.N, 0, in, c.N, 0, out, c.N, c.N);
-            g.rs = evp(c, s, j); g.rs_kind = SC_PLAIN;
-            if (j == lo && !bottom) { g.cs = c.LD[s] + (size_t)(m + 1) * c.N; g.cs_kind = SC_PLAIN; }
-            g1.push_back(g);
-            w = out;
-          }
-          if (j == hi) ends.push_back(ci);
-        }
-        b.gemm(ops, g1, 0);
-        for (int ci : ends) {
-          Chain& c = x->ch[ci];
-          const int m = (c.L - 1 - j) / ns;
+          const int m = c.nb - 1 - up;
+          if (m < m_min) continue;
           const bool bottom = (m == c.nb - 1);
           for (int s = 0; s < 2; ++s) {
             const size_t n2 = (size_t)c.N * c.N;
@@ -705,8 +736,9 @@ static void build_program(lqmc_ctx* x) {
           g2.push_back(mk(c.Tw[s], c.N, 0, ek, c.N, 0, Gp(c, s), c.N, c.N));
         }
       }
-      // right product W = E_K V(l) In; FP64 and independent of the wrap, so in FP64
-      // sweeps its tasks join the first wrap launch
+      // right product W = E_K V(l) In: all slices of a block at its end where E_K factors into directions
+      // of up to 16 sites; else FP64 and independent of the wrap, so in FP64 sweeps its tasks join the
+      // first wrap launch
       if (fp32) b.gemm(x->sweep_ops, g1, fp32);
       std::vector<int> bnd, ml, rvsel;
       for (int ci = 0; ci < nc; ++ci) {
@@ -714,8 +746,17 @@ static void build_program(lqmc_ctx* x) {
         if (t >= c.L) continue;
         const int l = c.L - 1 - t;
         const bool first = (t % ns == 0);
+        const bool end = (t + 1) % ns == 0 || t == c.L - 1;
+        if (end) bnd.push_back(ci);
         for (int s = 0; s < 2; ++s) {
           double*& w = wcur[ci * 2 + s];
+          if (Builder::chains(c)) {
+            const bool rid = rvcur[ci] < 0;
+            w = c.Wa[s];
+            if (end)
+              b.chain(kc, c, rid ? c.eye : c.RU[s], w, nullptr, evp(c, s, l + t % ns), rid ? nullptr : c.RD[s], -1, t % ns + 1);
+            continue;
+          }
           double* out = (first || w == c.Wb[s]) ? c.Wa[s] : c.Wb[s];
           const bool rid = rvcur[ci] < 0;
           const double* in = first ? (rid ? c.eye : c.RU[s]) : w;
@@ -725,10 +766,10 @@ static void build_program(lqmc_ctx* x) {
           g1.push_back(g);
           w = out;
         }
-        if ((t + 1) % ns == 0 || t == c.L - 1) bnd.push_back(ci);
       }
       b.gemm(x->sweep_ops, g1, 0);
       b.gemm(x->sweep_ops, g2, fp32);
+      b.chain(x->sweep_ops, kc);
       if (bnd.empty()) continue;
       for (int ci : bnd) {
         Chain& c = x->ch[ci];
@@ -763,7 +804,7 @@ static void run_ops(lqmc_ctx* x, const std::vector<Op>& ops, int measure, hipStr
     else if (op.kind == OP_GEMM) pk = PK_GEMM;
     else if (op.kind == OP_QR) pk = PK_QR;
     else if (op.kind == OP_SOLVE || op.kind == OP_TRSM) pk = PK_SOLVE;
-    else if (op.kind == OP_KRON || op.kind == OP_KRON_WIDE) pk = PK_KRON;
+    else if (op.kind == OP_KRON || op.kind == OP_KRON_WIDE || op.kind == OP_KRON_CHAIN) pk = PK_KRON;
     const bool rec = profile && pk == x->prof.kind;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (rec) {
@@ -775,6 +816,9 @@ static void run_ops(lqmc_ctx* x, const std::vector<Op>& ops, int measure, hipStr
     switch (op.kind) {
       case OP_GEMM: launch_gemm(op.fp32, op.nmax, reinterpret_cast<const GemmTask*>(d), op.count, op.ntiles, s); break;
       case OP_KRON: launch_kron(op.nmax, op.fp32, reinterpret_cast<const KronTask*>(d), op.count, op.ntiles, x->cus, s); break;
+      case OP_KRON_CHAIN:
+        launch_kron_chain(op.fp32, reinterpret_cast<const KronChainTask*>(d), op.count, op.ntiles, s);
+        break;
       case OP_KRON_WIDE:
         launch_kron_wide(op.nmax, reinterpret_cast<const KronTask*>(d), op.count, op.ntiles, op.threads, op.shmem, s);
         break;

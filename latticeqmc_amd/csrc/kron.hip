@@ -28,7 +28,8 @@ __device__ inline kr_v4d kr_mma(double a, double b, kr_v4d c) {
 }
 
 // Index of the task holding tile `tile` (tasks sorted by tile_base).
-__device__ inline int kr_task(const KronTask* __restrict__ tasks, int ntasks, int tile) {
+template <typename Task>
+__device__ inline int kr_task(const Task* __restrict__ tasks, int ntasks, int tile) {
   int lo = 0, hi = ntasks - 1;
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
@@ -234,6 +235,121 @@ void launch_kron(int right, int all16, const KronTask* d_tasks, int ntasks, int 
   else if (right) hipLaunchKernelGGL((k_kron<true, false>), dim3(grid), dim3(256), kron_shmem(), s, d_tasks, ntasks, ntiles);
   else if (all16) hipLaunchKernelGGL((k_kron<false, true>), dim3(grid), dim3(256), kron_shmem(), s, d_tasks, ntasks, ntiles);
   else hipLaunchKernelGGL((k_kron<false, false>), dim3(grid), dim3(256), kron_shmem(), s, d_tasks, ntasks, ntiles);
+}
+
+// ---- the left products of a stabilisation block -----------------------------------------------
+// Columns of X stay independent through left products, so a workgroup takes its 16 columns through all steps
+// in LDS (layout and matrix-core products of k_kron<false>, the same bits): X is read and C written once per
+// block instead of once per slice, and a block is one launch.  Bound by the matrix cores for many chains
+// (128 matrices of 256 sites, 8 steps: 113 us against 8 x 24 us) and by the steps' latency for few
+// (one 16 x 16 chain: 27 us against 8 launches of 6 us).
+template <bool F16>
+__global__ __launch_bounds__(256, F16 ? 4 : 3) void k_kron_chain(const KronChainTask* __restrict__ tasks, int ntasks) {
+  LQMC_DYNAMIC_LDS(double, vs);
+  double* const sc = vs + 16 * KR_AS;  // [2][256] scales, by the parity of the step
+  const int tile = blockIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readlane(tid >> 6, 0), li = lane & 15, lk = lane >> 4;
+  const KronChainTask tk = tasks[kr_task(tasks, ntasks, tile)];
+  const int t0 = (tile - tk.tile_base) * KR_T;
+  const int N = F16 ? 256 : tk.N, n1 = F16 ? 16 : tk.n1, n2 = F16 ? 16 : tk.n2;
+  const LQMC_GLOBAL double* X = gptr(tk.X);
+  const bool pre = tk.ks != nullptr, post = tk.rs != nullptr;
+  const LQMC_GLOBAL double* scg = gptr(pre ? tk.ks : tk.rs);
+  const bool has = (pre || post) && tid < N;
+  double nxt = has ? scg[tid] : 1.0;
+  {
+    double v[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+      int ap, bp, j;
+      kr_coords<false>(tid + 256 * u, ap, bp, j);
+      const bool ok = F16 || (ap < n1 && bp < n2 && t0 + j < N);
+      v[u] = ldg0(X, (size_t)(ap * n2 + bp) * N + t0 + j, ok);
+    }
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+      int ap, bp, j;
+      kr_coords<false>(tid + 256 * u, ap, bp, j);
+      vs[ap * KR_AS + bp * KR_BS + j] = v[u];
+    }
+  }
+  double ay[4], ax[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    ay[s] = gptr(tk.Ey)[li * 16 + 4 * s + lk];
+    ax[s] = gptr(tk.Ex)[li * 16 + 4 * s + lk];
+  }
+  const int col = t0 + li;
+  const double cv = tk.cs && col < N ? tk.cs[col] : 1.0;
+#pragma unroll 1
+  for (int step = 0; step < tk.steps; ++step) {
+    double* const sl = sc + 256 * (step & 1);
+    if (tid < N) sl[tid] = nxt;
+    if (has && step + 1 < tk.steps) nxt = scg[(long)(step + 1) * tk.stride + tid];
+    __syncthreads();
+    // the b' direction of this wavefront's a' blocks (in place)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      if (!F16 && wave + 8 * h >= n1) break;
+      kr_v4d acc[2];
+#pragma unroll
+      for (int q = 0; q < 2; ++q) acc[q] = kr_v4d{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+        if (F16 || 4 * s < n2) {
+#pragma unroll
+          for (int q = 0; q < 2; ++q) {
+            const int ap = wave + 8 * h + 4 * q, bp = 4 * s + lk;
+            const double kf = pre && (F16 || (ap < n1 && bp < n2)) ? sl[ap * n2 + bp] : 1.0;
+            acc[q] = kr_mma(ay[s], vs[ap * KR_AS + bp * KR_BS + li] * kf, acc[q]);
+          }
+        }
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) vs[(wave + 8 * h + 4 * q) * KR_AS + (lk + 4 * r) * KR_BS + li] = acc[q][r];
+    }
+    __syncthreads();
+    // the a' direction of this wavefront's b (in place, or to C after the last step)
+    const double cf = step == 0 ? cv : 1.0;
+    const bool end = step + 1 == tk.steps;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      if (!F16 && wave + 8 * h >= n2) break;
+      kr_v4d acc[2];
+#pragma unroll
+      for (int q = 0; q < 2; ++q) acc[q] = kr_v4d{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+        if (F16 || 4 * s < n1) {
+#pragma unroll
+          for (int q = 0; q < 2; ++q)
+            acc[q] = kr_mma(ax[s], vs[(4 * s + lk) * KR_AS + (wave + 8 * h + 4 * q) * KR_BS + li], acc[q]);
+        }
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int b = wave + 8 * h + 4 * q;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int a = lk + 4 * r;
+          const bool in = F16 || (a < n1 && b < n2);
+          const double rf = post && in ? sl[a * n2 + b] : 1.0;
+          const double v = rf * acc[q][r] * cf;
+          if (!end) vs[a * KR_AS + b * KR_BS + li] = v;
+          else if (in && (F16 || col < N)) gptr(tk.C)[(size_t)(a * n2 + b) * N + col] = v;
+        }
+      }
+    }
+    // the next step's first barrier orders these writes before its reads
+  }
+}
+
+size_t kron_chain_shmem() { return sizeof(double) * (16 * KR_AS + 2 * 256); }
+
+void launch_kron_chain(int all16, const KronChainTask* d_tasks, int ntasks, int ntiles, hipStream_t s) {
+  if (ntasks <= 0 || ntiles <= 0) return;
+  if (all16) hipLaunchKernelGGL(k_kron_chain<true>, dim3(ntiles), dim3(256), kron_chain_shmem(), s, d_tasks, ntasks);
+  else hipLaunchKernelGGL(k_kron_chain<false>, dim3(ntiles), dim3(256), kron_chain_shmem(), s, d_tasks, ntasks);
 }
 
 // ---- directions of up to 32 sites -------------------------------------------------------------
