@@ -38,6 +38,8 @@ size_t kron_wide_shmem(int n1, int n2);
 int gemm_class(const GemmTask& t);
 int gemm_tiles(int M, int N, int* tiles_n);
 void launch_qr_blocked(const QrTask* d, int n, int nmax, ChainState* st, unsigned* pub, int max_wg, hipStream_t s);
+void launch_qr_large(const QrTask* d, int n, int nmax, ChainState* st, hipStream_t s);
+int qr_large_limit();
 void launch_trsm(const TrsmTask* d, int n, int nmax, ChainState* st, hipStream_t s);
 void launch_solve(const SolveTask* d, int n, int nmax, ChainState* st, hipStream_t s);
 void launch_finish(int fp32, const FinishTask* d, int n, int nmax, ChainState* st, hipStream_t s);
@@ -823,7 +825,13 @@ static void run_ops(lqmc_ctx* x, const std::vector<Op>& ops, int measure, hipStr
         launch_kron_wide(op.nmax, reinterpret_cast<const KronTask*>(d), op.count, op.ntiles, op.threads, op.shmem, s);
         break;
       case OP_QR:
-        launch_qr_blocked(reinterpret_cast<const QrTask*>(d), op.count, op.nmax, x->d_state, x->d_qrpub, x->cus, s);
+        // N of 257 to 640: several workgroups per matrix, which hold a column block's rows in registers (more
+        // rows don't fit); a sweep of 12 slices against k_qr_blocked, 17x16: 1 chain 20.5 -> 13.0 ms,
+        // 128 chains 50.0 -> 46.3 ms; 24x24: 1 chain 73.8 -> 29.6 ms; 20x32: 16 chains 124 -> 59 ms.
+        if (op.nmax > 256 && op.nmax <= qr_large_limit())
+          launch_qr_large(reinterpret_cast<const QrTask*>(d), op.count, op.nmax, x->d_state, s);
+        else
+          launch_qr_blocked(reinterpret_cast<const QrTask*>(d), op.count, op.nmax, x->d_state, x->d_qrpub, x->cus, s);
         break;
       case OP_TRSM: launch_trsm(reinterpret_cast<const TrsmTask*>(d), op.count, op.nmax, x->d_state, s); break;
       case OP_SOLVE: launch_solve(reinterpret_cast<const SolveTask*>(d), op.count, op.nmax, x->d_state, s); break;

@@ -1512,19 +1512,9 @@ size_t trsm_shmem(int) { return sizeof(double) * (TRSM_B * QF_COLS + TRSM_B * TR
 // QR of n matrices (explicit Q formed).  N <= 256: the on-chip factorisation, at most
 // max_wg workgroups per launch (the compute units, so the two workgroups of a matrix are
 // resident together) with hand[2 n] (zero between launches) for the hand-over between them.
-// N up to 640: several workgroups per matrix, which hold a column block's rows in registers (more
-// rows don't fit); a sweep of 12 slices against k_qr_blocked, 17x16: 1 chain 20.5 -> 13.0 ms,
-// 128 chains 50.0 -> 46.3 ms; 24x24: 1 chain 73.8 -> 29.6 ms; 20x32: 16 chains 124 -> 59 ms.
 // Larger N: the blocked factorisation with the trailing matrix in global memory.
-int qr_large_limit();
-void launch_qr_large(const QrTask* d, int n, int nmax, ChainState* st, hipStream_t s);
-
 void launch_qr_blocked(const QrTask* d, int n, int nmax, ChainState* st, unsigned* hand, int max_wg, hipStream_t s) {
   if (n <= 0) return;
-  if (nmax > QO_NMAX && nmax <= qr_large_limit()) {
-    launch_qr_large(d, n, nmax, st, s);
-    return;
-  }
   if (nmax <= 64) {
     hipLaunchKernelGGL(k_qr_small, dim3(n), dim3(QU_THREADS), qr_small_shmem(), s, d, st);
   } else if (nmax <= QO_NMAX) {
