@@ -735,6 +735,28 @@ __device__ inline void qo_wait(unsigned* c, unsigned after, ChainState* st, int 
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
 }
 
+// a / b as the compiler's FP64 division forms it, without its scaling of operands and result: the
+// same quotient for operands and quotients well inside the exponent range.  qo_recip: 1 / b as that
+// division refines it; qo_quot: the quotient from it.
+__device__ inline double qo_recip(double b) {
+#ifdef LQMC_CPU_EMU
+  return 1.0 / b;
+#else
+  double r = __builtin_amdgcn_rcp(b);
+  r = fma(fma(-b, r, 1.0), r, r);
+  return fma(fma(-b, r, 1.0), r, r);
+#endif
+}
+__device__ inline double qo_quot(double a, double b, double r) {
+#ifdef LQMC_CPU_EMU
+  return a / b;
+#else
+  const double q = a * r;
+  return fma(fma(-b, q, a), r, q);
+#endif
+}
+__device__ inline double qo_div(double a, double b) { return qo_quot(a, b, qo_recip(b)); }
+
 // Q_P^T applied to one strip held in registers (rows j0 = 16 P .. 16 NS - 1; the panel's V,
 // explicit with unit diagonal and zeros above it, in vbuf; T in tbuf), NT >= NS row tiles held:
 // V^T X, which needs V alone, then X -= V (T^T (V^T X)).
@@ -782,7 +804,9 @@ __device__ inline void qo_apply(qo_acc_t (&acc)[NT], const double* vbuf, const d
 // V (explicit, unit diagonal, from the reflectors below the diagonal of A) and T (stored
 // transposed, since qo_apply applies I - V T_buf^T V^T) go to LDS once per workgroup, and a
 // wavefront skips the panels right of its columns, which leave them unchanged.  Q is written
-// once, at the end (the blocked k_qr_formq reads and writes its column block per panel).
+// once, at the end (the blocked k_qr_formq reads and writes its column block per panel).  Bound by the
+// panels' latency; with the next panel read ahead
+// 18 -> 13 us at N = 64, 56 -> 42 us for 512 matrices of 36 to 100 sites, 119 -> 114 us for 128 of 256.
 __global__ __launch_bounds__(QF_THREADS, 2) void k_qr_formq_onchip(const QrTask* __restrict__ tasks, int nblk) {
   const int gb = xcd_grouped_block();  // a matrix's column blocks on one XCD
   const QrTask tk = tasks[gb / nblk];
@@ -803,20 +827,30 @@ __global__ __launch_bounds__(QF_THREADS, 2) void k_qr_formq_onchip(const QrTask*
   for (int t = 0; t < 16; ++t)
 #pragma unroll
     for (int v = 0; v < 4; ++v) acc[t][v] = (16 * t + lk + 4 * v) == c ? 1.0 : 0.0;
-  for (int P = (c1 - 1) >> 4; P >= 0; --P) {
+  // a panel's V (this thread: column vc, rows j0 + vr + 16 u) and T are read from memory while the
+  // panel before it is applied
+  const int vr = tid >> 4, vc = tid & 15;
+  double av[16], tv;
+  auto fetch = [&](int P) {
+    const int j0 = P << 4, w = min(16, N - j0), jc = j0 + vc;
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+      const int r = j0 + vr + 16 * u;
+      if (u < NS - P) av[u] = ldg0(gptr(tk.A), (size_t)r * N + jc, r < N && vc < w && r > jc);
+    }
+    tv = ldg0(gptr(tk.Tt) + (size_t)P * 256, vc * 16 + vr, vr < w && vc < w);
+  };
+  const int Pl = (c1 - 1) >> 4;
+  fetch(Pl);
+  for (int P = Pl; P >= 0; --P) {
     const int j0 = P << 4, w = min(16, N - j0);
     __syncthreads();  // every wavefront is done with the previous panel's buffers
-    for (int e = tid; e < (QO_NMAX - j0) * 16; e += QF_THREADS) {
-      const int r = j0 + (e >> 4), cc = e & 15, jc = j0 + cc;
-      const bool in = r < N && cc < w;
-      const double a = ldg0(gptr(tk.A), (size_t)r * N + jc, in && r > jc);
-      vbuf[r * QO_PS + cc] = in ? (r > jc ? a : (r == jc ? 1.0 : 0.0)) : 0.0;
-    }
-    for (int e = tid; e < 256; e += QF_THREADS) {
-      const int i = e >> 4, j = e & 15;
-      tbuf[e] = (i < w && j < w) ? tk.Tt[(size_t)P * 256 + j * 16 + i] : 0.0;
-    }
+#pragma unroll
+    for (int u = 0; u < 16; ++u)
+      if (u < NS - P) vbuf[(j0 + vr + 16 * u) * QO_PS + vc] = u == 0 && vr == vc && vc < w ? 1.0 : av[u];
+    tbuf[tid] = tv;
     __syncthreads();
+    if (P > 0) fetch(P - 1);
     if (cs >= P && cs < NS) qo_apply<16>(acc, vbuf, tbuf, NS, P);
   }
   if (c < c1)
@@ -836,11 +870,15 @@ size_t qr_formq_onchip_shmem() { return sizeof(double) * ((size_t)QO_NMAX * QO_P
 // accumulator layout (row 16 t + l/16 + 4 v, column l%16 of lane l).  Row blocks of 16 from the
 // bottom: the block's band of R' goes to LDS, each wavefront forms Z[blk] - R'[blk, below]
 // Y'[below] on the matrix cores from its registers (the accumulator layout of Y' is the operand
-// layout of the product), the 16 x 16 diagonal systems are solved one lane per column through
-// LDS, and the block joins the registers.  Y is written once, permuted, at the end (the blocked
-// k_trsm_perm re-reads the solution below each block from global memory).
+// layout of the product), the 16 x 16 diagonal systems are solved one lane per column, and the
+// block joins the registers.  Y is written once, permuted, at the end (the blocked k_trsm_perm
+// re-reads the solution below each block from global memory).  Bound by the blocks' latency: with the
+// next band read ahead and the diagonal systems in registers, a wavefront's own columns each, 40 -> 15 us
+// at N = 64, 95 -> 57 us for 36 to 100 sites, 254 -> 203 us for 128 matrices of 256 (208 -> 160 for two).
 constexpr int TO_LD = QO_NMAX + 1;  // LDS row stride of the R' band
 
+// NT: row tiles held.
+template <int NT = 16>
 __global__ __launch_bounds__(QF_THREADS, 2) void k_trsm_onchip(const TrsmTask* __restrict__ tasks, int nblk,
                                                                ChainState* st) {
   const int gb = xcd_grouped_block();  // a matrix's column blocks on one XCD
@@ -860,55 +898,91 @@ __global__ __launch_bounds__(QF_THREADS, 2) void k_trsm_onchip(const TrsmTask* _
   const int c = c0 + wave * 16 + li;
   const bool cok = c < c1;
   bool zero = false;
-  qo_acc_t y[16];
+  qo_acc_t y[NT];
 #pragma unroll
-  for (int t = 0; t < 16; ++t) y[t] = qo_acc_t{0.0, 0.0, 0.0, 0.0};
-  for (int i = NS - 1; i >= 0; --i) {
-    // the band's columns i0 .. 16 NS - 1, zero past N (the products below read whole 16-column
-    // tiles, whose rows of Y' past N are zero: stale LDS there could hold a NaN)
-    const int i0 = i << 4, b = min(16, N - i0), nc = 16 * NS - i0;
-    __syncthreads();  // the previous block's reads of band and blk are done
-    for (int e = tid; e < 16 * nc; e += QF_THREADS) {
-      const int ii = e / nc, cc = i0 + e % nc;
-      band[ii * TO_LD + cc] = ldg0(Rg, (size_t)(i0 + ii) * N + cc, ii < b && cc < N);
+  for (int t = 0; t < NT; ++t) y[t] = qo_acc_t{0.0, 0.0, 0.0, 0.0};
+  // a block's band of R' (this thread: column bc, rows br + 2^(8 - sh) u) and right-hand sides are read
+  // from memory while the block below is solved; columns i0 .. 16 NS - 1, zero past N (the products read
+  // whole 16-column tiles, whose rows of Y' past N are zero: stale LDS there could hold a NaN)
+  const int sh = NS <= 4 ? 6 : (NS <= 8 ? 7 : 8);
+  const int bc = tid & ((1 << sh) - 1), br = tid >> sh;
+  double bv[NT], zv[4];
+  auto fetch = [&](int i) {
+    const int i0 = i << 4, b = min(16, N - i0);
+#pragma unroll
+    for (int u = 0; u < NT; ++u) {
+      const int ii = br + (u << (8 - sh));
+      if (u < (16 >> (8 - sh))) bv[u] = ldg0(Rg, (size_t)(i0 + ii) * N + bc, ii < b && bc >= i0 && bc < N);
     }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) zv[v] = ldg0(Zg, (size_t)(i0 + lk + 4 * v) * N + c, lk + 4 * v < b && cok);
+  };
+  fetch(NS - 1);
+  for (int i = NS - 1; i >= 0; --i) {
+    const int i0 = i << 4, b = min(16, N - i0);
+    __syncthreads();  // the previous block's reads of band are done
+#pragma unroll
+    for (int u = 0; u < NT; ++u)
+      if (u < (16 >> (8 - sh)) && bc >= i0 && bc < 16 * NS) band[(br + (u << (8 - sh))) * TO_LD + bc] = bc >= N && bc - i0 == br + (u << (8 - sh)) ? 1.0 : bv[u];
     qr_v4d acc;
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int row = lk + 4 * v;
-      acc[v] = ldg0(Zg, (size_t)(i0 + row) * N + c, row < b && cok);
-    }
+    for (int v = 0; v < 4; ++v) acc[v] = zv[v];
     __syncthreads();
+    if (i > 0) fetch(i - 1);
     // acc -= R'[blk, j] Y'_j for the blocks j below (A lane l: R'[i0 + l%16][16 j + l/16 + 4 v])
 #pragma unroll
-    for (int j = 0; j < 16; ++j) {
+    for (int j = 0; j < NT; ++j) {
       if (j <= i || j >= NS) continue;
 #pragma unroll
       for (int v = 0; v < 4; ++v) acc = qr_mma(-band[li * TO_LD + 16 * j + lk + 4 * v], y[j][v], acc);
     }
+    // the 16 x 16 system of my wavefront's columns, one lane per column, the solution in registers
 #pragma unroll
     for (int v = 0; v < 4; ++v) blk[(lk + 4 * v) * QF_COLS + wave * 16 + li] = acc[v];
-    __syncthreads();
-    if (tid < QF_COLS) {
-      for (int ii = b - 1; ii >= 0; --ii) {
-        double sv = blk[ii * QF_COLS + tid];
-        for (int kk = ii + 1; kk < b; ++kk) sv -= band[ii * TO_LD + i0 + kk] * blk[kk * QF_COLS + tid];
-        const double d = band[ii * TO_LD + i0 + ii];
-        if (d == 0.0) zero = true;
-        blk[ii * QF_COLS + tid] = sv / d;
-      }
+    qr_wave_sync();
+    // (rows past N: zero right-hand side, diagonal one)
+    const double* dg = band + i0;
+    const double dl = dg[li * TO_LD + li], rl = qo_recip(dl);  // of row li
+    if (dl == 0.0) zero = true;
+    double rs[16], ds[16];  // of every row, in scalar registers
+#pragma unroll
+    for (int ii = 0; ii < 16; ++ii) {
+      rs[ii] = qo_readlane(rl, ii);
+      ds[ii] = qo_readlane(dl, ii);
     }
-    __syncthreads();
+    if (lane < 16) {
+      double xs[16];
+#pragma unroll
+      for (int ii = 0; ii < 16; ++ii) xs[ii] = blk[ii * QF_COLS + wave * 16 + li];
+      // up to 8 tiles, a row's entries are read while the row below is solved (the fences keep the reads of
+      // all rows from being gathered first, for want of registers)
+      double row[2][16];
+#pragma unroll
+      for (int ii = 15; ii >= 0; --ii) {
+        if (NT <= 8 && ii > 0) {
+#pragma unroll
+          for (int kk = ii; kk < 16; ++kk) row[(ii - 1) & 1][kk] = dg[(ii - 1) * TO_LD + kk];
+        }
+        double sv = xs[ii];
+#pragma unroll
+        for (int kk = ii + 1; kk < 16; ++kk) sv -= (NT <= 8 ? row[ii & 1][kk] : dg[ii * TO_LD + kk]) * xs[kk];
+        xs[ii] = qo_quot(sv, ds[ii], rs[ii]);
+        qr_sched_fence();
+      }
+#pragma unroll
+      for (int ii = 0; ii < 16; ++ii) blk[ii * QF_COLS + wave * 16 + li] = xs[ii];
+    }
+    qr_wave_sync();
     qr_v4d sol;
 #pragma unroll
     for (int v = 0; v < 4; ++v) sol[v] = blk[(lk + 4 * v) * QF_COLS + wave * 16 + li];
 #pragma unroll
-    for (int t = 0; t < 16; ++t)
+    for (int t = 0; t < NT; ++t)
       if (t == i) y[t] = sol;
   }
   if (cok)
 #pragma unroll
-    for (int t = 0; t < 16; ++t)
+    for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         const int r = 16 * t + lk + 4 * v;
@@ -928,19 +1002,6 @@ struct QoShared {
   int vs;               // doubles of one V
 };
 
-// a / b as the compiler's FP64 division forms it, without its scaling of operands and result: the
-// same quotient for operands and quotients well inside the exponent range.
-__device__ inline double qo_div(double a, double b) {
-#ifdef LQMC_CPU_EMU
-  return a / b;
-#else
-  double r = __builtin_amdgcn_rcp(b);
-  r = fma(fma(-b, r, 1.0), r, r);
-  r = fma(fma(-b, r, 1.0), r, r);
-  const double q = a * r;
-  return fma(fma(-b, q, a), r, q);
-#endif
-}
 // sqrt(x) likewise, x well inside the exponent range.
 __device__ inline double qo_sqrt(double x) {
 #ifdef LQMC_CPU_EMU
@@ -1544,9 +1605,10 @@ void launch_qr_blocked(const QrTask* d, int n, int nmax, ChainState* st, unsigne
 void launch_trsm(const TrsmTask* d, int n, int nmax, ChainState* st, hipStream_t s) {
   if (n <= 0) return;
   const int nblk = (nmax + QF_COLS - 1) / QF_COLS;
-  if (nmax <= QO_NMAX)
-    hipLaunchKernelGGL(k_trsm_onchip, dim3(n * nblk), dim3(QF_THREADS), trsm_onchip_shmem(), s, d, nblk, st);
-  else
+  if (nmax <= QO_NMAX) {
+    auto k = nmax <= 64 ? k_trsm_onchip<4> : nmax <= 128 ? k_trsm_onchip<8> : k_trsm_onchip<16>;
+    hipLaunchKernelGGL(k, dim3(n * nblk), dim3(QF_THREADS), trsm_onchip_shmem(), s, d, nblk, st);
+  } else
     hipLaunchKernelGGL(k_trsm_perm, dim3(n * nblk), dim3(QF_THREADS), trsm_shmem(nmax), s, d, nblk, st);
 }
 
